@@ -648,3 +648,57 @@ def test_prefill_backward_empty_sides(Sq, Skv):
     assert torch.count_nonzero(dq.float()).item() == 0 and not torch.isnan(dq.float()).any()
     assert torch.count_nonzero(dk.float()).item() == 0 and not torch.isnan(dk.float()).any()
     assert torch.count_nonzero(dv.float()).item() == 0 and not torch.isnan(dv.float()).any()
+
+
+# One shape or more per kernel and index mapping that the host's size rule can pick for calls too
+# small for one walk of all keys per row block (32-key tiles, 32-row units, (batch, KV head) counts of
+# 1, 2, 4, multiples of 8 and others): remainders of 1 and 31 rows and keys on both sides of a tile.
+SPLIT_CASES = [
+    # dtype, B, Sq, Skv, H, Hkv, causal, off
+    ("bf16", 1, 33, 1057, 8, 1, 1, 1024),    # eight key parts, one (batch, KV head)
+    ("bf16", 1, 1, 1025, 2, 2, 1, 1024),     # more waves than the last round has tiles
+    ("bf16", 3, 31, 95, 6, 2, 1, 64),        # four key parts, six (batch, KV head)s
+    ("bf16", 1, 65, 3, 4, 4, 0, 0),          # fewer keys than a tile, no mask
+    ("bf16", 2, 40, 70, 10, 2, 1, -9),       # rows that see no key, group of 5
+    ("bf16", 8, 97, 97, 32, 4, 1, 0),        # shared tiles, two key parts
+    ("bf16", 3, 352, 400, 32, 4, 1, 48),     # the same, 12 (batch, KV head)s
+    ("bf16", 24, 97, 129, 32, 4, 1, 32),     # shared tiles, one key part
+    ("bf16", 2, 33, 2049, 16, 4, 0, 0),      # long keys, no mask
+    ("f32", 1, 33, 1057, 8, 1, 1, 1024),
+    ("f32", 3, 31, 95, 6, 2, 1, 64),
+    ("f32", 2, 40, 70, 10, 2, 1, -9),
+    ("f32", 16, 97, 65, 32, 4, 0, 0),        # two key parts
+    ("f32", 1, 513, 513, 8, 4, 1, 0),        # the paired order's odd last round
+]
+
+
+@pytest.mark.parametrize("case", SPLIT_CASES)
+def test_prefill_key_split_kinds(case):
+    dtype, Bn, Sq, Skv, H, Hkv, causal, off = case
+    q = draw((Bn, Sq, H, 64), 21, dtype)
+    k = draw((Bn, Skv, Hkv, 64), 22, dtype)
+    v = draw((Bn, Skv, Hkv, 64), 23, dtype)
+    args = (dev(q, TD[dtype]), dev(k, TD[dtype]), dev(v, TD[dtype]))
+    o, lse = B.gqa_prefill_lse(*args, scale=0.125, causal=bool(causal), seq_offset=off)
+    assert_close(host(o), O.gqa_prefill(q, k, v, 0.125, bool(causal), off), TOL[dtype], f"prefill {case}")
+    ref, got = O.gqa_prefill_lse(q, k, 0.125, bool(causal), off), host(lse)
+    seen = np.isfinite(ref)
+    assert np.array_equal(got == -np.inf, ~seen)
+    assert np.max(np.abs(got[seen] - ref[seen])) <= TOL[dtype]  # absolute, as for the lse above
+    again = B.gqa_prefill(*args, scale=0.125, causal=bool(causal), seq_offset=off)
+    assert torch.equal(again, o)
+
+
+def test_prefill_f32_wide_kv_rows():
+    # K/V rows 2^24 elements apart: past the 32-bit range of a tile's buffer descriptor
+    Sq, Skv, H, Hkv, rs = 37, 39, 4, 2, 1 << 24
+    q, k, v = (draw((1, s, h, 64), 24 + i, "f32") for i, (s, h) in enumerate(((Sq, H), (Skv, Hkv), (Skv, Hkv))))
+    buf = torch.empty((Skv - 1) * rs + 2 * Hkv * 64, device="cuda")
+
+    def wide(x, off):
+        w = buf.as_strided((1, Skv, Hkv, 64), (rs, rs, 64, 1), off)
+        w.copy_(dev(x))
+        return w
+
+    o = B.gqa_prefill(dev(q), wide(k, 0), wide(v, Hkv * 64), scale=0.125, seq_offset=2)
+    assert_close(host(o), O.gqa_prefill(q, k, v, 0.125, True, 2), TOL["f32"])
