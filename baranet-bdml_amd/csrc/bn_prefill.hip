@@ -991,30 +991,42 @@ __global__ __launch_bounds__(64 * KW, 2) void prefill_f32_ks_kernel(PrefillParam
 }
 
 // Which kernel takes a call.  `units`: (head, 32 query rows) pieces of the
-// work, nt: 32-key tiles of the longest row block.  The lines lie where the
-// measured times cross (us, graph replay, 32 query / 4 KV heads; "rows": the
-// kernel above, whose waves walk all keys of their rows; s4/s8: one unit per
-// workgroup over 4/8 waves; sh/sh2: four heads, 1/2 key parts):
+// work, nt: 32-key tiles of the longest row block, even: every row block sees
+// about as many keys (no mask, or as many cached keys as new rows).  The lines
+// lie where the measured times cross (us, graph replay; "rows": the kernel
+// above, whose waves walk all keys of their rows; s4/s8: one unit per
+// workgroup over 4/8 waves; sh/sh2: four heads, 1/2 key parts; 32 query heads
+// over 4 KV heads unless said):
 //   units   64, nt 131 (64 rows of 4160 keys)   rows 71.5  s4 22.0  s8 17.6  sh2 44.6
 //   units  256, nt 136 (256 rows of 4352)       rows 73.5  s4 25.5  s8 20.6  sh2 46.8
 //   units   32, nt  16 (16 rows of 512)         rows 14.5  s4  6.3  s8  6.5  sh2  9.8
 //   units  512, nt  16 (B=1 S=512)              rows 15.9  s4  7.7  s8 11.1  sh2 10.4
 //   units  640, nt 104 (B=2, 300 rows of 3300)  rows 60.8  s4 35.9  s8 42.0  sh2 38.0
-//   units 1024, nt  32 (B=1 S=1024)             rows 24.3  s4 15.0           sh2 15.7
-//   units 1024, nt   4 (B=8 S=128)              rows  9.8  s4  8.8           sh2  7.1  sh 6.9
+//   units  896, nt  14 (B=2 S=438)              rows 14.6  s4 10.5           sh2 10.1  sh 11.7
+//   units  992, nt  31 (S=992)                  rows 23.5  s4 15.7           sh2 16.1  sh 20.1
+//   units 1024, nt   4 (B=8 S=105)              rows  9.9  s4  8.9           sh2  7.2  sh  7.1
 //   units 1600, nt  25 (B=2 S=777)              rows 21.7  s4 19.4           sh2 15.7  sh 18.1
-//   units 2048, nt  64 (B=1 S=2048)             rows 40.3                    sh2 30.3  sh 36.8
+//   units 1792, nt   8 (B=7 S=235)              rows 12.4                    sh2 10.4  sh  9.5
+//   units 2048, nt  64 (S=2048)                 rows 40.3                    sh2 30.3  sh 36.8
+//   units 2560, nt  20 (B=4 S=622)              rows 20.1                    sh2 18.0  sh 16.6
 //   units 4096, nt  32 (B=4 S=1024)             rows 31.9                    sh2 29.9  sh 28.2
-//   units 4096, nt 128 (B=1 S=4096)             rows 99.4                    sh2 87.9  sh 90.6
+//   units 4096, nt 128 (S=4096)                 rows 99.4                    sh2 87.9  sh 90.6
 //   units 5376, nt  56 (B=3 S=1777)             rows 53.5                    sh2 57.2  sh 56.1
 //   units 8192, nt  64 (B=4 S=2048)             rows 81.4                    sh2 91.5  sh 84.8
-// With every row block about as long (no mask, or as many cached keys as new
-// rows) the row kernel of 8-head groups has no tail to lose and holds from
-// 2048 units (2048 rows of 16384 keys: 277 against sh2 288).  Groups that are
-// no multiple of 4 have no shared form; there the row kernel (one head per
-// workgroup) holds above 1024 units (8 heads, B=4 S=2048: 34.2 against s4 39.4;
-// B=1 S=4096 52.8 against 36.5), or 512 of equal length (B=2 S=2048 without
-// mask 27.9 against 32.2; B=1 27.0 against 18.7).
+//   units 19840, nt 31 (B=20 S=988)             rows 120.6                   sh2 137.4 sh 117.2
+//   even: units 2048, nt 512 (2048 rows of 16384) rows 277                   sh2 288
+//         units 3584, nt  20 (B=16, 213 of 639)   rows 28.8                  sh2 31.9  sh 29.5
+// Groups of 4 (the row kernel has twice the workgroups there):
+//   units 1984, nt  62 (S=1957)                 rows 29.6                    sh2 27.1
+//   units 2240, nt  20 (B=7 S=630)              rows 15.7                    sh2 16.4  sh 16.2
+//   units 3072, nt  96 (S=3053)                 rows 53.6                              sh 58.8
+//   units 3200, nt  20 (B=5 S=634)              rows 19.3                    sh2 20.0  sh 17.7
+//   even: units 1232, nt  31 (B=7, 330 of 990)  rows 19.9                    sh2 20.6  sh 21.6
+//         units 2048, nt 256 (2048 of 8192)     rows 155                     sh2 142
+// Groups that are no multiple of 4 have no shared form; there the row kernel
+// (one head per workgroup) holds above 1024 units (8 heads, B=4 S=2048: 34.2
+// against s4 39.4; S=4096 52.8 against 36.5), or 512 even ones (B=2 S=2048
+// without mask 27.9 against 32.2; B=1 27.0 against 18.7).
 // fp32 (matrix-core time alone counts) is always key-split: s8/s4/two waves
 // S=512 21.0/19.6/30.4, B=4 S=512 72.4/56.1/50.2, S=2048 170.8/148.1/159.5,
 // B=2 S=2048 339/286/281, 256 rows of 4352 76.0/85.9/153.9.
@@ -1028,8 +1040,17 @@ KsKind ks_kind(int dtype, int batch, int n_kv_heads, int group, int seq_q, int s
   const KsKind few = units <= 256 && nt > 32 ? KsKind::split8 : KsKind::split4;
   if (dtype == BN_F32) return units <= (nt >= 64 ? 2048 : 1536) ? few : KsKind::split2;
   if (group % 4 != 0) return units > (even ? 512 : 1024) ? KsKind::none : few;
-  if (units >= 8192 || (nt >= 32 && units >= (group == 8 && even ? 2048 : 5120))) return KsKind::none;
-  return units >= 3072 ? KsKind::shared : units >= 1024 ? KsKind::shared2 : few;
+  const bool wide = group >= 8;
+  if (units < (even ? 768 : nt <= 16 ? 640 : 1024)) return few;
+  if (nt <= 4) return KsKind::shared;
+  if (nt < 32) {
+    if (even && (wide ? units >= 3200 && nt > 16 : units >= 1024 && nt > 8)) return KsKind::none;
+    if (!wide && nt > 16 && units > 2048 && units < 3072) return KsKind::none;
+    return units > (nt <= 8 ? 1024 : 2048) ? KsKind::shared : KsKind::shared2;
+  }
+  if (even && (wide ? units >= 2048 : units >= 1024 && nt < 64)) return KsKind::none;
+  if (units <= (wide ? 3072 : 2048)) return KsKind::shared2;
+  return wide && units < 5120 ? KsKind::shared : KsKind::none;
 }
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
