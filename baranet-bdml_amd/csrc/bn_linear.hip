@@ -18,6 +18,7 @@
 // (the transposed view of an [n, k] matrix) through linear_gemv_t_kernel,
 // one launch with the epilogue and no partials.
 #include <algorithm>
+#include <utility>
 
 #include "bn_common.hpp"
 
@@ -208,6 +209,270 @@ __global__ __launch_bounds__(256, 2) void linear_kernel(LinParams p, RopeFreqs f
     } else {
       rope4(v, gm, gn, p, fr);
       store4<T>((T *)p.y + gm * p.y_rs + gn, v);
+    }
+  }
+}
+
+// ------------------------------------------------------- bf16, many rows
+// y = x @ w on v_mfma_f32_16x16x32_bf16 with the rotation in the epilogue.  4
+// waves own 32 MF x 32 NF outputs (a quarter each); stages of 64 k go through
+// two LDS buffers, loaded into registers two stages ahead.  D = w^T x^T: a
+// lane holds 4 consecutive columns of one row, so a rotation pair is its own.
+// What bounds it is the one wave per SIMD that a prompt's few tiles leave: LDS
+// writes (64 bytes a clock), reads, loads and products add up unless each is
+// spread between the others, so a stage's stores, fragment reads and loads are
+// dealt evenly among its products (issued in clusters: 33.5 against 28.4 us at
+// 2048 x 2560, K 2048 without rotation; without loads and stores 22, products
+// alone 18).  Rotation angles cost one hardware sine and cosine per row and
+// frequency and tile (LDS table); per element with sincosf, and its arguments
+// read by vector loads, they took 12 of 65 us.
+// Measured (graph replay) against the 64x64-tile kernel above: 2048 x 2560, K
+// 2048 with rotation 65 -> 33.9 us (633 TFLOP/s; the library product alone 34,
+// before its separate rotation), 8192 rows 190 -> 101 (850 TFLOP/s), 512 rows
+// 25.6 -> 18.8, 64 rows 14.0 -> 11.7; 2048 x 11264 214 -> 114.  Rotating the
+// tiles' first stage apart (for the memory channels) cost 5-60%.
+template <class F, int... I>
+__device__ __forceinline__ void unroll_seq(F &&f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void unroll(F &&f) {
+  unroll_seq(f, std::make_integer_sequence<int, N>{});
+}
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+// sine and cosine of x by the hardware's, which take turns: x / 2pi split in
+// two floats, so the reduction adds no error to them
+__device__ __forceinline__ void sincos_turns(float x, float *sn, float *cs) {
+  constexpr float kHi = 0.15915493667125702f, kLo = 6.4206382e-09f;  // 1 / 2pi
+  const float hi = x * kHi;
+  const float lo = fmaf(x, kLo, fmaf(x, kHi, -hi));
+  const float t = __builtin_amdgcn_fractf(hi) + lo;
+  *sn = __builtin_amdgcn_sinf(t);
+  *cs = __builtin_amdgcn_cosf(t);
+}
+
+template <int MF, int NF, int OCC>
+__global__ __launch_bounds__(256, OCC) void linear_mn_kernel(LinParams p, RopeFreqs fr) {
+  constexpr int BM = 32 * MF, BN = 32 * NF, KT = 64;
+  constexpr int WP = BN + 8, XP = KT + 8;       // LDS pitches, elements
+  constexpr int WC = BN / 8, NWC = KT * WC / 256, NXC = BM * (KT / 8) / 256;
+  constexpr int WS = KT * WP, XS = BM * XP;     // one stage
+  __shared__ __attribute__((aligned(16))) bf16_t smem[2 * (WS + XS)];
+  __shared__ float fq[kMaxRopePairs];  // the rotation's frequencies
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, g = lane >> 4;
+  const int m_off = 16 * MF * (wave >> 1), n_off = 16 * NF * (wave & 1);
+  // tile order: an XCD's workgroups (ids equal mod 8) take a run of tiles, 8
+  // row tiles by columns
+  const int tm = (p.m + BM - 1) / BM, tn = (p.n + BN - 1) / BN, nt = tm * tn;
+  const int per = (nt + 7) / 8;
+  const int t = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || t >= nt) return;
+  const int band = t / (8 * tn), bh = min(8, tm - 8 * band), r = t - band * 8 * tn;
+  const int m0 = (8 * band + r % bh) * BM, n0 = (r / bh) * BN;
+  const bf16_t *X = (const bf16_t *)p.x + (int64_t)m0 * p.x_rs, *W = (const bf16_t *)p.w;
+
+  auto rsrc = [&](const bf16_t *base, int64_t bytes) __attribute__((always_inline)) {
+    const uint64_t a = (uint64_t)base;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+    return __builtin_amdgcn_make_buffer_rsrc((void *)(((uint64_t)hi << 32) | lo), (short)0,
+                                             __builtin_amdgcn_readfirstlane((int)bytes), 0x00020000);
+  };
+  const int nst = (p.k + KT - 1) / KT;
+  constexpr int OOB = 0x7ffffff0;
+  int wofs[NWC], xofs[NXC];
+#pragma unroll
+  for (int i = 0; i < NWC; ++i) {
+    const int c = tid + 256 * i, col = n0 + (c % WC) * 8;
+    wofs[i] = col < p.n ? ((c / WC) * (int)p.w_rs + col) * 2 : OOB;
+  }
+#pragma unroll
+  for (int i = 0; i < NXC; ++i) {
+    const int c = tid + 256 * i;
+    xofs[i] = ((c >> 3) * (int)p.x_rs + (c & 7) * 8) * 2;
+  }
+  const int64_t xrange = (int64_t)min(BM, p.m - m0) * p.x_rs * 2;
+  struct Regs {
+    u32x4_t w[NWC], x[NXC];
+  };
+  Regs ra, rb;  // the next two stages
+  auto klen = [&](int st) { return max(0, min(KT, p.k - st * KT)); };  // past k: empty, nothing read
+  auto gload_w = [&](Regs &q, int st) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t r = rsrc(W + (int64_t)st * KT * p.w_rs, (int64_t)klen(st) * p.w_rs * 2);
+#pragma unroll
+    for (int i = 0; i < NWC; ++i)
+      q.w[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, wofs[i], 0, 0));
+  };
+  auto gload_x = [&](Regs &q, int st) __attribute__((always_inline)) {
+    const int kl = klen(st);
+    const __amdgpu_buffer_rsrc_t r = rsrc(X + st * KT, kl > 0 ? xrange : 0);
+    const int past = (tid & 7) * 8 < kl ? 0 : 1 << 30;  // columns past k are the next row's
+#pragma unroll
+    for (int i = 0; i < NXC; ++i)
+      q.x[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, xofs[i] + past, 0, 0));
+  };
+  // k row of a stage -> LDS row: a transposed read of lane group g takes k
+  // 8g..8g+3 (then 8g+4..8g+7) of a 32-k block, as x's 16-byte fragments
+  // hold them; its 16 rows are adjacent in LDS (pitch BN + 8: no conflicts)
+  auto wrow = [](int k) { return (k & ~31) + 16 * ((k >> 2) & 1) + 4 * ((k >> 3) & 3) + (k & 3); };
+  auto lstore_w = [&](const Regs &q, int buf) __attribute__((always_inline)) {
+    bf16_t *const ws = smem + buf * (WS + XS);
+#pragma unroll
+    for (int i = 0; i < NWC; ++i) {
+      const int c = tid + 256 * i;
+      *(u32x4_t *)(ws + wrow(c / WC) * WP + (c % WC) * 8) = q.w[i];
+    }
+  };
+  auto lstore_x = [&](const Regs &q, int buf) __attribute__((always_inline)) {
+    bf16_t *const xs = smem + buf * (WS + XS) + WS;
+#pragma unroll
+    for (int i = 0; i < NXC; ++i) *(u32x4_t *)(xs + ((tid >> 3) + 32 * i) * XP + (tid & 7) * 8) = q.x[i];
+  };
+  f32x4_t acc[NF][MF];
+#pragma unroll
+  for (int f = 0; f < NF; ++f)
+#pragma unroll
+    for (int i = 0; i < MF; ++i) acc[f][i] = f32x4_t{};
+  const int tr_off = (4 * g + (l16 >> 2)) * WP + n_off + 4 * (l16 & 3);
+  const int x_off = (m_off + l16) * XP + 8 * g;
+  struct Frags {
+    bf16x8_t w[NF], x[MF];
+  };
+  auto fread = [&](Frags &q, int buf, int kk) __attribute__((always_inline)) {
+    const bf16_t *const ws = smem + buf * (WS + XS), *const xs = ws + WS;
+#pragma unroll
+    for (int i = 0; i < MF; ++i) q.x[i] = *(const bf16x8_t *)(xs + x_off + 16 * i * XP + 32 * kk);
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      const bf16_t *wp = ws + 32 * kk * WP + tr_off + 16 * f;
+      const bf16x4_t lo = tr16(wp), hi = tr16(wp + 16 * WP);
+      q.w[f] = bf16x8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    }
+  };
+  auto mac = [&](const Frags &q) __attribute__((always_inline)) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int i = 0; i < MF; ++i)
+        acc[f][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q.w[f], q.x[i], acc[f][i], 0, 0, 0);
+  };
+  constexpr int NR = 2 * NF + MF, NM = NF * MF;  // LDS reads and products of 32 k
+  Frags f0, f1;
+  gload_w(ra, 0);
+  gload_x(ra, 0);
+  gload_w(rb, 1);
+  gload_x(rb, 1);
+  // by scalar loads: the arguments lie in host memory, and a vector load of
+  // them from every workgroup at its end took 9 us of a 38 us call
+  if (n0 < p.rope_cols && wave == 0)
+    for (int q = 0; 2 * q < p.head_dim; q += 16) {
+      float v = 0.f;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) v = lane == j ? fr.f[q + j] : v;
+      if (lane < 16) fq[q + lane] = v;
+    }
+  lstore_w(ra, 0);
+  lstore_x(ra, 0);
+  gload_w(ra, 2);
+  gload_x(ra, 2);
+  __syncthreads();
+  fread(f0, 0, 0);
+  lstore_w(rb, 1);
+  auto spread = [&](auto nst_, auto nld_) __attribute__((always_inline)) {
+    unroll<NM>([&](auto ic) __attribute__((always_inline)) {
+      constexpr int i = decltype(ic)::value, NS = decltype(nst_)::value, NG = decltype(nld_)::value;
+      constexpr int nr = (i + 1) * NR / NM - i * NR / NM, ns = (i + 1) * NS / NM - i * NS / NM;
+      constexpr int ng = (i + 1) * NG / NM - i * NG / NM;
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      if constexpr (nr > 0) __builtin_amdgcn_sched_group_barrier(0x100, nr, 0);
+      if constexpr (ns > 0) __builtin_amdgcn_sched_group_barrier(0x200, ns, 0);
+      if constexpr (ng > 0) __builtin_amdgcn_sched_group_barrier(0x020, ng, 0);
+    });
+  };
+  // stage s, its first 32 k's fragments in f0.  Their products run with the
+  // second's fragment reads, the stores of stage s+1's x (its w went in one
+  // phase earlier) and the loads of stage s+3's w into the registers w left;
+  // after the barrier the second's products with stage s+1's first reads,
+  // stage s+2's w stores (the buffer's reads are over) and stage s+3's x loads
+  auto stage = [&](Regs &q, Regs &q2, int s) __attribute__((always_inline)) {
+    fread(f1, s & 1, 1);
+    mac(f0);
+    lstore_x(q, (s + 1) & 1);
+    gload_w(q, s + 3);
+    spread(std::integral_constant<int, NXC>{}, std::integral_constant<int, NWC>{});
+    __syncthreads();
+    fread(f0, (s + 1) & 1, 0);
+    mac(f1);
+    lstore_w(q2, s & 1);
+    gload_x(q, s + 3);
+    spread(std::integral_constant<int, NWC>{}, std::integral_constant<int, NXC>{});
+  };
+  for (int s = 0; s < nst; s += 2) {
+    stage(rb, ra, s);
+    if (s + 1 < nst) stage(ra, rb, s + 1);
+  }
+
+  // acc[f][i][e]: row m_off + 16i + l16, column n_off + 16f + 4g + e.  The
+  // tile's rotation angles go through an LDS table [row][frequency] (the
+  // staging buffers are free), one sine and cosine per row and frequency.
+  const int hq = p.head_dim >> 1;
+  const int tp = hq + 1;  // table pitch: rows on different banks
+  const bool table = n0 < p.rope_cols && BM * tp * 8 <= 2 * (WS + XS) * 2;  // uniform
+  float2 *const sc = reinterpret_cast<float2 *>(smem);
+  if (table) {
+    __syncthreads();  // the last stage's reads ahead
+    int row = tid / hq, q = tid - row * hq;
+    const int drow = 256 / hq, dq = 256 - drow * hq;
+    while (row < BM) {
+      float2 v;
+      sincos_turns((float)(p.pos0 + m0 + row) * fq[q], &v.x, &v.y);
+      sc[row * tp + q] = v;
+      row += drow;
+      q += dq;
+      if (q >= hq) {
+        q -= hq;
+        ++row;
+      }
+    }
+    __syncthreads();
+  }
+  // branch-free (a wave's reads of one column group go out together, stores
+  // past the edges fall outside the descriptor)
+  const __amdgpu_buffer_rsrc_t ry = rsrc((const bf16_t *)p.y + (int64_t)m0 * p.y_rs,
+                                         (int64_t)min(BM, p.m - m0) * p.y_rs * 2);
+#pragma unroll
+  for (int f = 0; f < NF; ++f) {
+    const int gn = n0 + n_off + 16 * f + 4 * g;
+    const bool r0 = gn < p.rope_cols, r1 = gn + 2 < p.rope_cols;
+    float2 ta[MF], tb[MF];
+    if (table) {
+      const float2 *sa = sc + (m_off + l16) * tp + (r0 ? (gn % p.head_dim) >> 1 : 0);
+      const float2 *sb = sc + (m_off + l16) * tp + (r1 ? ((gn + 2) % p.head_dim) >> 1 : 0);
+#pragma unroll
+      for (int i = 0; i < MF; ++i) {
+        ta[i] = sa[16 * i * tp];
+        tb[i] = sb[16 * i * tp];
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < MF; ++i) {
+        const float pos = (float)(p.pos0 + m0 + m_off + 16 * i + l16);
+        if (r0) sincos_turns(pos * fq[(gn % p.head_dim) >> 1], &ta[i].x, &ta[i].y);
+        if (r1) sincos_turns(pos * fq[((gn + 2) % p.head_dim) >> 1], &tb[i].x, &tb[i].y);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < MF; ++i) {
+      const float4 x = make_float4(acc[f][i][0], acc[f][i][1], acc[f][i][2], acc[f][i][3]);
+      const float s0 = r0 ? ta[i].x : 0.f, c0 = r0 ? ta[i].y : 1.f, s1 = r1 ? tb[i].x : 0.f, c1 = r1 ? tb[i].y : 1.f;
+      typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+      const u32x2_t v = {(uint32_t)f32_to_bf16(x.x * c0 - x.y * s0) | ((uint32_t)f32_to_bf16(x.x * s0 + x.y * c0) << 16),
+                         (uint32_t)f32_to_bf16(x.z * c1 - x.w * s1) | ((uint32_t)f32_to_bf16(x.z * s1 + x.w * c1) << 16)};
+      const int off = ((m_off + 16 * i + l16) * (int)p.y_rs + gn) * 2;
+      __builtin_amdgcn_raw_buffer_store_b64(v, ry, gn < p.n ? off : OOB, 0, 0);
     }
   }
 }
@@ -859,6 +1124,58 @@ int nt_run(const bn_view *x, const bn_view *w, const bn_view *y, int rope_cols, 
   return BN_OK;
 }
 
+// Which bf16 calls linear_mn_kernel takes, and its tile.  A workgroup per CU
+// at a time: a tile of MF x NF fragments costs c microseconds per 64 k, and
+// ceil(tiles / 256) of them follow each other (fitted within 10% on 37 shapes
+// of 16-8192 rows, K 1024-5632; e.g. 2048 x 2560, K 2048: 128x128 tiles are
+// 320 = two rounds, 44.2 us; 128x160 are 256 = one, 33.9; 3000 rows: 43.8
+// against 48.1).  Few rows keep the split-k kernel, whose slabs fill the chip
+// where K is long (us, split-k / here: K 2048, 32 x 2560 10.3 / 11.5, 64 x
+// 1536 11.0 / 11.6, 64 x 2560 14.0 / 11.7, 64 x 11264 19.0 / 14.9; K 1024, 40
+// x 1536 7.8 / 8.4, 100 x 1536 10.2 / 8.4; K 4096, 250 x 1536 20.3 / 23.7,
+// 200 x 3072 25.0 / 26.4, 250 x 3072 26.9 / 26.6, 700 x 1536 35.3 / 30.6;
+// K 5632, 320 x 2048 27.9 / 31.7).
+bool mn_takes(int m, int n, int k, int64_t x_rs, int64_t w_rs, int64_t y_rs) {
+  constexpr int64_t kMaxRs = 1 << 21;  // 160 rows of a tile stay below 2^30 bytes
+  const int64_t least = 48 + (k > 2048 ? (k - 2048) / 8 : 0);
+  return k > 0 && m >= 48 && (int64_t)m * n >= 2560 * least && x_rs < kMaxRs && w_rs < kMaxRs && y_rs < kMaxRs;
+}
+int mn_run(const bn_view *x, const bn_view *w, const bn_view *y, int rope_cols, int position_offset,
+           int head_dim, const RopeFreqs &fr, hipStream_t s) {
+  LinParams p = {};
+  p.x = (const bf16_t *)x->data + x->offset;
+  p.w = (const bf16_t *)w->data + w->offset;
+  p.y = (bf16_t *)y->data + y->offset;
+  p.x_rs = x->stride_h; p.w_rs = w->stride_h; p.y_rs = y->stride_h;
+  p.m = y->h; p.n = w->w; p.k = x->w;
+  p.rope_cols = rope_cols; p.head_dim = rope_cols ? head_dim : 2; p.pos0 = position_offset;
+  struct Tile {
+    int mf, nf;
+    float c;
+    void (*kernel)(LinParams, RopeFreqs);
+  };
+  static const Tile tiles[] = {
+      {4, 5, .66f, linear_mn_kernel<4, 5, 2>}, {4, 4, .55f, linear_mn_kernel<4, 4, 2>},
+      {4, 3, .45f, linear_mn_kernel<4, 3, 2>}, {2, 5, .48f, linear_mn_kernel<2, 5, 2>},
+      {2, 4, .39f, linear_mn_kernel<2, 4, 2>}, {2, 3, .31f, linear_mn_kernel<2, 3, 2>},
+      {2, 2, .21f, linear_mn_kernel<2, 2, 3>}, {1, 2, .14f, linear_mn_kernel<1, 2, 3>}};
+  const Tile *best = nullptr;
+  int64_t best_n = 0;
+  float best_c = 0.f;
+  for (const Tile &t : tiles) {
+    const int64_t nt = (int64_t)((p.m + 32 * t.mf - 1) / (32 * t.mf)) * ((p.n + 32 * t.nf - 1) / (32 * t.nf));
+    const float c = (float)((nt + 255) / 256) * t.c;
+    if (!best || c < best_c) {
+      best = &t;
+      best_n = nt;
+      best_c = c;
+    }
+  }
+  hipLaunchKernelGGL(best->kernel, dim3((unsigned)((best_n + 7) / 8 * 8)), dim3(256), 0, s, p, fr);
+  BN_LAUNCH_CHECK();
+  return BN_OK;
+}
+
 // output-major w (linear_gemv_t_kernel): shapes and the rotation table are
 // checked by linear_run; this checks the layout the kernel reads
 int gemv_t_run(const bn_view *x, const bn_view *w, const bn_view *y, int rope_cols,
@@ -1041,6 +1358,8 @@ int linear_run(const bn_view *x, const bn_view *w, const bn_view *y, int rope_co
     return fail(BN_ERR_UNSUPPORTED, std::string(op) + ": problem too large");
   if ((st = ensure_device())) return st;
   hipStream_t s = as_stream(stream);
+  if (dt == BN_BF16 && epi == EPI_PLAIN && !k_dst && mn_takes(m, n, k, x->stride_h, w->stride_h, y->stride_h))
+    return mn_run(x, w, y, rope_cols, position_offset, head_dim, fr, s);
   void *ws = workspace;
   bool own = false;
   if (need && !ws) {

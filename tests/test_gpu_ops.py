@@ -528,3 +528,37 @@ def test_argmax_rows_ties_nan_strided():
     um = torch.empty((3, 1), dtype=torch.int32, device="cuda")
     B.call("bn_argmax", V(ud), V(um), S0)
     np.testing.assert_array_equal(host(um)[:, 0], [_argmax_sequential(row) for row in u])
+
+
+# bf16 prompts: one shape or more for every tile that the host's cost rule can pick, with ragged row and
+# column tiles, k below and past a stage of 64, positions past 4096 and head widths on both sides of
+# the rotation table's limit.
+MANY_ROWS_BF16 = [
+    # M, K, N, rope_cols, offset, head_dim
+    (2047, 136, 2560, 2304, 0, 64),     # 128 x 160
+    (1500, 72, 2568, 2304, 4000, 64),   # 128 x 128
+    (1025, 64, 2568, 0, 0, 64),         # 128 x 96, no rotation
+    (1000, 8, 2560, 2560, 3, 128),      # 64 x 160 of less than a stage
+    (1100, 200, 2048, 1984, 7, 64),     # 64 x 128
+    (640, 2048, 2048, 2016, 100, 96),   # 64 x 96, head width no power of two
+    (330, 1992, 2568, 2304, 0, 512),    # 64 x 64, angles per element
+    (129, 520, 1024, 512, 9, 2),        # 32 x 64
+    (48, 64, 2560, 2304, 16000, 64),    # the fewest rows
+]
+
+
+@pytest.mark.parametrize("case", MANY_ROWS_BF16)
+def test_linear_rope_bf16_many_rows(case):
+    M, K, N, rc, off, hd = case
+    rc = rc // hd * hd
+    r = rng(66)
+    x = bf16_round(r.standard_normal((M, K)).astype(np.float32))
+    w = bf16_round((r.standard_normal((K, N)) / np.sqrt(K)).astype(np.float32))
+    yb = torch.full((M, N + 16), 7.0, device="cuda", dtype=torch.bfloat16)
+    xb = torch.full((M, K + 24), float("nan"), device="cuda", dtype=torch.bfloat16)
+    xb[:, 8:8 + K] = dev(x, torch.bfloat16)
+    B.linear_rope(xb[:, 8:8 + K], dev(w, torch.bfloat16), yb[:, 8:8 + N], rope_cols=rc, position_offset=off,
+                  head_dim=hd)
+    got = host(yb)
+    assert_close(got[:, 8:8 + N], O.linear_rope(x, w, rc, off, hd, 1e4), BF16_TOL, f"many rows {case}")
+    assert np.all(got[:, :8] == 7.0) and np.all(got[:, 8 + N:] == 7.0)
