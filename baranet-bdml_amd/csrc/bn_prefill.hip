@@ -11,7 +11,7 @@
 // 4 x 32*RT query rows of one (batch, head), or 32 rows of a group's heads;
 // each wave owns 32*RT rows and walks all their keys.  Key blocks of 64 are
 // staged in LDS with the next blocks' global loads in flight while the current
-// block is computed.  Smaller bf16 calls, and all fp32 ones, split the keys of
+// block is computed.  Smaller bf16 calls, and most fp32 ones, split the keys of
 // 32 query rows over the waves of a workgroup instead (ks_kind).
 //
 // Per wave and key tile the score tile is computed transposed,
@@ -41,6 +41,7 @@ typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
+constexpr int BM = 128;  // query rows per workgroup (fp32 row kernel)
 constexpr int BN = 64;   // keys per LDS block
 constexpr int HD = 64;   // head_dim
 
@@ -84,6 +85,47 @@ __device__ __forceinline__ int key_end(const PrefillParams &p, int last_row) {
   long e = (long)last_row + p.seq_offset + 1;
   if (e < 0) e = 0;
   return e < p.seq_kv ? (int)e : p.seq_kv;
+}
+
+// Online-softmax update of one 64-key block for this lane's query.
+// s[kt][i] holds key kb + kt*32 + (i/4)*8 + hf*4 + (i%4).
+__device__ __forceinline__ void softmax_block(f32x16_t (&s)[2], float &m, float &l,
+                                              f32x16_t (&o)[2], float c, bool need_mask,
+                                              int kb, int hf, long qlimit, int seq_kv) {
+  if (need_mask) {
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int key = kb + kt * 32 + (i >> 2) * 8 + hf * 4 + (i & 3);
+        if (key >= seq_kv || (long)key > qlimit) s[kt][i] = -INFINITY;
+      }
+  }
+  float mx = s[0][0];
+#pragma unroll
+  for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[kt][i]);
+  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+  const float m_new = fmaxf(m, mx);
+  const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
+  const float mc = m_use * c;
+  const float alpha = __builtin_amdgcn_exp2f(m * c - mc);  // m = -inf -> 0
+  float rs = 0.f;
+#pragma unroll
+  for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float e = __builtin_amdgcn_exp2f(fmaf(s[kt][i], c, -mc));
+      s[kt][i] = e;
+      rs += e;
+    }
+  l = l * alpha + rs;  // per half-wave partial; halves are summed at the end
+  m = m_new;
+#pragma unroll
+  for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
 }
 
 // ------------------------------------------------------------------ bf16
@@ -804,10 +846,150 @@ __global__ __launch_bounds__(64 * HW * KW, OCC) void prefill_bf16_ks_kernel(Pref
 }
 
 // ------------------------------------------------------------------- fp32
+constexpr int KP32 = HD + 4;  // 272 B pitch
+constexpr int VP32 = BN + 4;
+
+__global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillParams p) {
+  // double-buffered K and V^T blocks: one barrier per block
+  __shared__ __attribute__((aligned(16))) float Ks2[2][BN * KP32];
+  __shared__ __attribute__((aligned(16))) float Vt2[2][HD * VP32];
+
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int r32 = lane & 31, hf = lane >> 5;
+  // a (batch, KV head) group's heads and row tiles on one XCD: its K/V is
+  // read from HBM once, then from that XCD's L2
+  const Work w = decode_work_xcd(p);
+  const float *Q = (const float *)p.q + w.b * p.q_bs + (int64_t)w.h * HD;
+  const float *K = (const float *)p.k + w.b * p.kv_bs + (int64_t)w.g * HD;
+  const float *V = (const float *)p.v + w.b * p.kv_bs + (int64_t)w.g * HD;
+  float *O = (float *)p.o + w.b * p.o_bs + (int64_t)w.h * HD;
+
+  const int q_wave0 = w.mt * BM + wave * 32;
+  const int qrow = q_wave0 + r32;
+  const bool row_ok = qrow < p.seq_q;
+
+  // k-slot (hf, t) of the QK^T contraction is d = hf*32 + t
+  float qreg[32];
+#pragma unroll
+  for (int t = 0; t < 32; t += 4) {
+    float4 v4 = row_ok ? *(const float4 *)(Q + (int64_t)qrow * p.q_rs + hf * 32 + t)
+                       : make_float4(0.f, 0.f, 0.f, 0.f);
+    qreg[t] = v4.x; qreg[t + 1] = v4.y; qreg[t + 2] = v4.z; qreg[t + 3] = v4.w;
+  }
+
+  const int wg_last = min(w.mt * BM + BM, p.seq_q) - 1;
+  const int kend = key_end(p, wg_last);
+  const int nblk = (kend + BN - 1) / BN;
+  const int wave_last = min(q_wave0 + 31, p.seq_q - 1);
+  const int wave_kend = (wave_last < q_wave0) ? 0 : key_end(p, wave_last);
+  const long qlimit = p.causal ? (long)qrow + p.seq_offset : (long)p.seq_kv;
+
+  float4 kreg[4], vreg[4];
+  auto gload = [&](int kb) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int idx = tid + 256 * c, key = idx >> 4, dc = idx & 15;
+      const int kk = kb + key;
+      if (kk < p.seq_kv) {
+        kreg[c] = *(const float4 *)(K + (int64_t)kk * p.kv_rs + dc * 4);
+        vreg[c] = *(const float4 *)(V + (int64_t)kk * p.kv_rs + dc * 4);
+      } else {
+        kreg[c] = make_float4(0.f, 0.f, 0.f, 0.f);
+        vreg[c] = make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+    }
+  };
+  auto lstore = [&](int buf) {
+    float *Ks = Ks2[buf], *Vt = Vt2[buf];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int idx = tid + 256 * c, key = idx >> 4, dc = idx & 15;
+      *(float4 *)(Ks + key * KP32 + dc * 4) = kreg[c];
+      Vt[(dc * 4 + 0) * VP32 + key] = vreg[c].x;
+      Vt[(dc * 4 + 1) * VP32 + key] = vreg[c].y;
+      Vt[(dc * 4 + 2) * VP32 + key] = vreg[c].z;
+      Vt[(dc * 4 + 3) * VP32 + key] = vreg[c].w;
+    }
+  };
+
+  float m = -INFINITY, l = 0.f;
+  f32x16_t o[2] = {f32x16_t{}, f32x16_t{}};
+
+  // block blk is computed from buffer blk & 1 while block blk + 1 (loaded
+  // one block earlier) is stored into the other buffer, whose last reads were
+  // in block blk - 1, before the previous barrier
+  if (nblk > 0) {
+    gload(0);
+    lstore(0);
+  }
+  __syncthreads();
+  if (nblk > 1) gload(BN);
+  for (int blk = 0; blk < nblk; ++blk) {
+    const int kb = blk * BN, buf = blk & 1;
+    if (kb < wave_kend) {  // wave-uniform
+      const float *Ks = Ks2[buf], *Vt = Vt2[buf];
+    f32x16_t s[2];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      s[kt] = f32x16_t{};
+      const float *krow = Ks + (kt * 32 + r32) * KP32 + hf * 32;
+#pragma unroll
+      for (int t = 0; t < 32; t += 4) {
+        const float4 a = *(const float4 *)(krow + t);
+        s[kt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, qreg[t], s[kt], 0, 0, 0);
+        s[kt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, qreg[t + 1], s[kt], 0, 0, 0);
+        s[kt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, qreg[t + 2], s[kt], 0, 0, 0);
+        s[kt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, qreg[t + 3], s[kt], 0, 0, 0);
+      }
+    }
+    const bool need_mask =
+        (kb + BN > p.seq_kv) || (p.causal && (long)kb + BN - 1 > (long)q_wave0 + p.seq_offset);
+    softmax_block(s, m, l, o, p.c, need_mask, kb, hf, qlimit, p.seq_kv);
+
+    // register i of s[kt] is k-slot hf of key kt*32 + (i/4)*8 + hf*4 + i%4
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int gi = 0; gi < 4; ++gi) {
+        const int kbase = kt * 32 + gi * 8 + hf * 4;
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt) {
+          const float4 a = *(const float4 *)(Vt + (dt * 32 + r32) * VP32 + kbase);
+          o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, s[kt][4 * gi], o[dt], 0, 0, 0);
+          o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, s[kt][4 * gi + 1], o[dt], 0, 0, 0);
+          o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, s[kt][4 * gi + 2], o[dt], 0, 0, 0);
+          o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, s[kt][4 * gi + 3], o[dt], 0, 0, 0);
+        }
+      }
+    }
+    if (blk + 1 < nblk) {
+      lstore(buf ^ 1);
+      if (blk + 2 < nblk) gload(kb + 2 * BN);
+    }
+    __syncthreads();
+  }
+
+  const float lt = l + __shfl_xor(l, 32, 64);
+  const float inv = lt > 0.f ? 1.0f / lt : 0.f;
+  if (p.lse && hf == 0 && row_ok)
+    p.lse[((int64_t)w.b * p.n_heads + w.h) * p.seq_q + qrow] = row_lse(m * p.c, lt);
+  if (row_ok) {
+    float *orow = O + (int64_t)qrow * p.o_rs;
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+      for (int gi = 0; gi < 4; ++gi) {
+        const int d0 = dt * 32 + gi * 8 + hf * 4;
+        *(float4 *)(orow + d0) = make_float4(o[dt][4 * gi] * inv, o[dt][4 * gi + 1] * inv,
+                                             o[dt][4 * gi + 2] * inv, o[dt][4 * gi + 3] * inv);
+      }
+  }
+}
+
+// --------------------------------------------------------- fp32, keys split
 // The same split on v_mfma_f32_32x32x2f32 (64 cycles each: 64 of them per
 // 32-key tile and unit, so matrix-core time is all that counts and one wave
-// walking a 512-key row took 27 of the former one-wave-per-row-block kernel's
-// 43 us).  One (head, 32 query rows) unit per workgroup, its tiles dealt to KW
+// walking a 512-key row takes 27 of the row kernel's 43 us).  One (head, 32 query rows) unit per workgroup, its tiles dealt to KW
 // waves, no barrier before the merge: a wave stages its own K tile in LDS
 // (rows of 272 B) one tile ahead and reads V straight from memory -- P^T is
 // the PV product's B operand as the scores left it, so an A operand is two
@@ -818,9 +1000,7 @@ __global__ __launch_bounds__(64 * HW * KW, OCC) void prefill_bf16_ks_kernel(Pref
 // blocks): B=1 S=512 H=32 44.9 -> 17.2 us, S=2048 211 -> 148, B=4 S=2048 596
 // -> 544 (126 TFLOP/s, 82% of what a large fp32 product reaches), 256 rows
 // behind 4096 333 -> 76.
-// WIDE: row strides past a 32-bit tile range (2^24 elements and up) take
-// 64-bit addresses.
-template <int KW, bool WIDE>
+template <int KW>
 __global__ __launch_bounds__(64 * KW, 2) void prefill_f32_ks_kernel(PrefillParams p) {
   constexpr int KP = HD + 4;  // K row and O row pitch, floats
   constexpr int TILE = 32 * KP;
@@ -853,19 +1033,11 @@ __global__ __launch_bounds__(64 * KW, 2) void prefill_f32_ks_kernel(PrefillParam
     return __builtin_amdgcn_make_buffer_rsrc((void *)(((uint64_t)hi << 32) | lo), (short)0, nrec,
                                              0x00020000);
   };
-  const int row4 = WIDE ? 0 : 4 * (int)p.kv_rs;  // bytes
+  const int row4 = 4 * (int)p.kv_rs;  // bytes
   const int koff = (lane >> 4) * row4 + (lane & 15) * 16;  // 4 rows of 256 bytes per load
   const int voff = 4 * hf * row4 + r32 * 8;
   u32x4_t kr[8];
   auto gload_k = [&](int t) __attribute__((always_inline)) {
-    if constexpr (WIDE) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int row = 32 * t + 4 * j + (lane >> 4);
-        kr[j] = t < nt && row < p.seq_kv ? *(const u32x4_t *)(K + row * p.kv_rs + (lane & 15) * 4) : u32x4_t{};
-      }
-      return;
-    }
     const __amdgpu_buffer_rsrc_t r = rsrc(K, t);
 #pragma unroll
     for (int j = 0; j < 8; ++j)
@@ -888,13 +1060,7 @@ __global__ __launch_bounds__(64 * KW, 2) void prefill_f32_ks_kernel(PrefillParam
     for (int j = 0; j < 8; ++j) *(u32x4_t *)(kl + (4 * j + (lane >> 4)) * KP + (lane & 15) * 4) = kr[j];
     // this tile's V: key slot (hf, i) of the P V contraction is key 8(i/4) + 4hf + i%4
     float2 vr[16];
-    if constexpr (WIDE) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int row = 32 * t + 8 * (i >> 2) + 4 * hf + (i & 3);
-        vr[i] = row < p.seq_kv ? *(const float2 *)(V + row * p.kv_rs + 2 * r32) : make_float2(0.f, 0.f);
-      }
-    } else {
+    {
       const __amdgpu_buffer_rsrc_t r = rsrc(V, t);
 #pragma unroll
       for (int i = 0; i < 16; ++i)
@@ -1027,9 +1193,12 @@ __global__ __launch_bounds__(64 * KW, 2) void prefill_f32_ks_kernel(PrefillParam
 // (one head per workgroup) holds above 1024 units (8 heads, B=4 S=2048: 34.2
 // against s4 39.4; S=4096 52.8 against 36.5), or 512 even ones (B=2 S=2048
 // without mask 27.9 against 32.2; B=1 27.0 against 18.7).
-// fp32 (matrix-core time alone counts) is always key-split: s8/s4/two waves
-// S=512 21.0/19.6/30.4, B=4 S=512 72.4/56.1/50.2, S=2048 170.8/148.1/159.5,
-// B=2 S=2048 339/286/281, 256 rows of 4352 76.0/85.9/153.9.
+// fp32 (matrix-core time alone counts): rows/s8/s4/two waves S=512 44.9/21.0/
+// 19.6/30.4, B=4 S=512 60.6/72.4/56.1/50.2, S=2048 211/171/148/160, B=2 S=2048
+// 311/339/286/281 and without mask 567/582/531/572.  Rows of more than 2560
+// keys on average keep the row kernel's order of sums: the split's differs from
+// it by 1.1e-6 (relative, over the output) at 2000 keys and by 2.1e-6 at 4352
+// (it is the nearer one to 64 bits, 1.1e-6 against 2.4e-6).
 enum class KsKind { none, shared, shared2, split2, split4, split8 };
 KsKind ks_kind(int dtype, int batch, int n_kv_heads, int group, int seq_q, int seq_kv, int causal,
                int seq_offset) {
@@ -1038,7 +1207,11 @@ KsKind ks_kind(int dtype, int batch, int n_kv_heads, int group, int seq_q, int s
   const int64_t nt = ((causal ? std::min<int64_t>(seq_kv, seen) : seq_kv) + 31) / 32;
   const bool even = !causal || seq_offset >= seq_q;
   const KsKind few = units <= 256 && nt > 32 ? KsKind::split8 : KsKind::split4;
-  if (dtype == BN_F32) return units <= (nt >= 64 ? 2048 : 1536) ? few : KsKind::split2;
+  if (dtype == BN_F32) {
+    const int64_t first = causal ? std::max<int64_t>((int64_t)seq_offset + 1, 0) : seq_kv;  // by the first row
+    if (first + 32 * nt > 2 * 2560 + 32 || (!causal && units >= 4096)) return KsKind::none;
+    return units <= (nt >= 64 ? 2048 : 1536) ? few : KsKind::split2;
+  }
   if (group % 4 != 0) return units > (even ? 512 : 1024) ? KsKind::none : few;
   const bool wide = group >= 8;
   if (units < (even ? 768 : nt <= 16 ? 640 : 1024)) return few;
@@ -1107,7 +1280,7 @@ static int prefill_impl(int dtype, const void *q, const void *k, const void *v, 
   // a group's heads over 32 rows per workgroup; config 2 +6%, config 5 +3%)
   const int group = n_heads / n_kv_heads;
   const bool packed = dtype == BN_BF16 && (group == 8 || group == 4);
-  const int rows_per_wg = packed || dtype == BN_F32 ? 32 : 4 * 32 * rt16;
+  const int rows_per_wg = packed ? 32 : dtype == BN_BF16 ? 4 * 32 * rt16 : BM;
   const int n_mt = (seq_q + rows_per_wg - 1) / rows_per_wg;
   const int64_t n_wg = (int64_t)batch * (packed ? n_kv_heads : n_heads) * n_mt;
   if (n_wg > 0x7fffffff) return fail(BN_ERR_UNSUPPORTED, std::string(op) + ": problem too large");
@@ -1126,7 +1299,10 @@ static int prefill_impl(int dtype, const void *q, const void *k, const void *v, 
   p.lse = lse;
   p.snake = 0;
   hipStream_t s = as_stream(stream);
-  const KsKind ks = ks_kind(dtype, batch, n_kv_heads, group, seq_q, seq_kv, causal, seq_offset);
+  // (a tile of K/V rows is fetched through a 32-bit buffer range)
+  const KsKind ks = kv_row_stride >= ((int64_t)1 << 24)
+                        ? KsKind::none
+                        : ks_kind(dtype, batch, n_kv_heads, group, seq_q, seq_kv, causal, seq_offset);
   if (ks != KsKind::none) {
     const int rows = (seq_q + 31) / 32, ng = batch * n_kv_heads;
     const int n_hu = dtype == BN_BF16 && (ks == KsKind::shared || ks == KsKind::shared2) ? group / 4 : group;
@@ -1140,14 +1316,12 @@ static int prefill_impl(int dtype, const void *q, const void *k, const void *v, 
     // fp32: only where every workgroup is resident at once (two per CU)
     p.snake = dtype == BN_BF16 || n_items <= 512;
     if (dtype == BN_F32) {
-      if (kv_row_stride >= ((int64_t)1 << 24))
-        hipLaunchKernelGGL((prefill_f32_ks_kernel<4, true>), grid, dim3(256), 0, s, p);
-      else if (ks == KsKind::split8)
-        hipLaunchKernelGGL((prefill_f32_ks_kernel<8, false>), grid, dim3(512), 0, s, p);
+      if (ks == KsKind::split8)
+        hipLaunchKernelGGL(prefill_f32_ks_kernel<8>, grid, dim3(512), 0, s, p);
       else if (ks == KsKind::split4)
-        hipLaunchKernelGGL((prefill_f32_ks_kernel<4, false>), grid, dim3(256), 0, s, p);
+        hipLaunchKernelGGL(prefill_f32_ks_kernel<4>, grid, dim3(256), 0, s, p);
       else
-        hipLaunchKernelGGL((prefill_f32_ks_kernel<2, false>), grid, dim3(128), 0, s, p);
+        hipLaunchKernelGGL(prefill_f32_ks_kernel<2>, grid, dim3(128), 0, s, p);
     } else if (ks == KsKind::shared)
       hipLaunchKernelGGL((prefill_bf16_ks_kernel<4, 1, 4>), grid, dim3(256), 0, s, p);
     else if (ks == KsKind::shared2)
@@ -1156,7 +1330,9 @@ static int prefill_impl(int dtype, const void *q, const void *k, const void *v, 
       hipLaunchKernelGGL((prefill_bf16_ks_kernel<1, 4, 3>), grid, dim3(256), 0, s, p);
     else
       hipLaunchKernelGGL((prefill_bf16_ks_kernel<1, 8, 2>), grid, dim3(512), 0, s, p);
-  } else if (packed && group == 8)
+  } else if (dtype == BN_F32)
+    hipLaunchKernelGGL(prefill_f32_kernel, dim3((unsigned)n_wg), dim3(256), 0, s, p);
+  else if (packed && group == 8)
     hipLaunchKernelGGL((prefill_bf16_kernel<2, kOcc, true>), dim3((unsigned)n_wg), dim3(256), 0, s, p);
   else if (packed)
     hipLaunchKernelGGL((prefill_bf16_kernel<1, kOcc, true>), dim3((unsigned)n_wg), dim3(256), 0, s, p);

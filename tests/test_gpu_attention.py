@@ -665,6 +665,7 @@ SPLIT_CASES = [
     ("bf16", 24, 97, 129, 32, 4, 1, 32),     # shared tiles, one key part
     ("bf16", 2, 33, 2049, 16, 4, 0, 0),      # long keys, no mask
     ("f32", 1, 33, 1057, 8, 1, 1, 1024),
+    ("f32", 1, 33, 2500, 4, 1, 1, 2467),     # long rows: the row kernel
     ("f32", 3, 31, 95, 6, 2, 1, 64),
     ("f32", 2, 40, 70, 10, 2, 1, -9),
     ("f32", 16, 97, 65, 32, 4, 0, 0),        # two key parts
