@@ -19,7 +19,8 @@
 //   * every lane group keeps its own running (max, sum, acc) per head, updated
 //     once per tile of NT keys, and the groups, waves and chunks are merged
 //     with the log-sum-exp rule: in-wave by shuffles, in-workgroup through LDS,
-//     across chunks by a small combine kernel over (m, l, acc) partials.
+//     across chunks over (m, l, acc) partials, by a small combine kernel (fp32)
+//     or by a cache's last split to finish (bf16).
 // Scores live in the log2 domain: s = (q.k) * scale*log2(e), p = exp2(s - m).
 
 #include <algorithm>
@@ -99,6 +100,10 @@ struct DecodeParams {
   // unit's records and writes the output in the same launch; null: the
   // records are left for a combine
   uint32_t *cnt = nullptr;
+  // split whole-cache kernel: two arrival words per (sequence, KV head) below
+  // arrive_end (any contents before the launch), and the launch's 48-bit tag
+  unsigned long long *arrive_end = nullptr;
+  unsigned long long tag = 0;
 };
 
 // WV waves per workgroup; MODE:
@@ -345,379 +350,22 @@ __global__ __launch_bounds__(64 * WV) void decode_split_kernel(DecodeParams p) {
   }
 }
 
-// bf16 cache: matrix-core version.  Per wave, tiles of 32 keys:
+// bf16 caches run on the matrix cores.  Per wave, tiles of 32 keys:
 //   S^T[key][head] = K[key][:] . Q[head][:]   two v_mfma_f32_16x16x32_bf16 per
-//     16 keys; the K tile is the A operand straight from HBM (lane: key l%16,
-//     16 bytes of d), the G query heads are the B operand columns (padded to 16);
+//     16 keys; the K tile is the A operand (lane: key l%16, 16 bytes of d), the
+//     G query heads are the B operand columns (padded to 16);
 //   online softmax per head column (4 keys per lane, 4 lane groups);
-//   O^T[d][head] += V^T[d][key] . P^T[key][head]  one MFMA per 16 d; V^T comes
-//     from a per-wave LDS tile written transposed, P^T straight from registers.
-// The next tile's K/V loads are issued before the current tile is computed.
+//   O^T[d][head] += V^T[d][key] . P^T[key][head]  one MFMA per 16 d; V^T by
+//     transposed LDS reads, P^T straight from registers.
 typedef __bf16 dbf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 dbf16x4_t __attribute__((ext_vector_type(4)));
 typedef float df32x4_t __attribute__((ext_vector_type(4)));
 constexpr int TK = 32;   // keys per wave tile
-constexpr int VTP = 36;  // V^T LDS pitch (elements): conflict-free writes and b64 reads
-
-constexpr int NBUF = 2;  // register tile buffers in turn
-// register budget for 3 waves per SIMD
-template <int G>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
-void decode_bf16_mfma_kernel(DecodeParams p) {
-  // per-wave V^T tile; after the wave's last tile the same bytes hold its
-  // (acc) merge values, so the workgroup needs no second LDS array
-  __shared__ __attribute__((aligned(16))) bf16_t Vt[4][HD * VTP];
-  __shared__ float red_m[4][G], red_l[4][G];
-  static_assert(G * HD * sizeof(float) <= HD * VTP * sizeof(bf16_t), "merge area");
-
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int l16 = lane & 15, grp = lane >> 4;
-  const int split = blockIdx.x % p.n_split;
-  const int bg = blockIdx.x / p.n_split;
-  const int b = bg / p.n_kv_heads, g = bg % p.n_kv_heads;
-
-  int len = p.lens[b];
-  len = len < 0 ? 0 : (len > p.max_len ? p.max_len : len);
-  const int k_begin = split * p.chunk;
-  if (k_begin >= len) return;  // the combine kernel ignores chunks past len
-  const int k_end = min(k_begin + p.chunk, len);
-  const int ntiles = (k_end - k_begin + TK - 1) / TK;
-
-  const int64_t kv_rs = p.kv_rs;
-  const bf16_t *Kb = (const bf16_t *)p.k + b * p.kv_bs + g * p.kv_hs + 8 * grp;
-  const bf16_t *Vb = (const bf16_t *)p.v + b * p.kv_bs + g * p.kv_hs + 8 * grp;
-
-  // B operand of S^T: column l16 = query head g*G + l16 (zero past G), d = 8grp + 32t + 0..7
-  dbf16x8_t qb[2];
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    if (l16 < G)
-      qb[t] = *(const dbf16x8_t *)((const bf16_t *)p.q +
-                                   ((int64_t)b * p.n_heads + g * G + l16) * HD + 8 * grp + 32 * t);
-    else
-      qb[t] = dbf16x8_t{};
-  }
-
-  // NBUF register tile buffers used in turn: while one tile is computed, the
-  // loads of the other NBUF-1 (and the refill of this one) are in flight
-  uint4 kr[NBUF][2][2], vr[NBUF][2][2];  // [buffer][16-key half u][d half t]; lane: key 16u + l16
-  // Branch-free loads: a key past the end reads the last valid key instead
-  // (its score is masked to -inf, so P = 0 multiplies finite cache data).  A
-  // conditional load would make the compiler wait for every outstanding load
-  // at the first use, serialising the two buffers.
-  auto gload = [&](int buf, int kb) {
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int key = min(kb + 16 * u + l16, k_end - 1);
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        kr[buf][u][t] = *(const uint4 *)(Kb + (int64_t)key * kv_rs + 32 * t);
-        vr[buf][u][t] = *(const uint4 *)(Vb + (int64_t)key * kv_rs + 32 * t);
-      }
-    }
-  };
-
-  float m = -INFINITY, l = 0.f;
-  df32x4_t o[4] = {df32x4_t{}, df32x4_t{}, df32x4_t{}, df32x4_t{}};
-  bf16_t *vt = Vt[wave];
-  const float c = p.c;
-
-  auto compute = [&](int buf, int kb) {
-    // V tile -> LDS, transposed: vt[d][key], d = 8grp + 32t + e, key = 16u + l16.
-    // The tile is private to this wave; LDS operations of a wave complete in order.
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const uint4 vv = vr[buf][u][t];
-        const uint32_t w4[4] = {vv.x, vv.y, vv.z, vv.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          vt[(8 * grp + 32 * t + 2 * e) * VTP + 16 * u + l16] = (bf16_t)(w4[e] & 0xffffu);
-          vt[(8 * grp + 32 * t + 2 * e + 1) * VTP + 16 * u + l16] = (bf16_t)(w4[e] >> 16);
-        }
-      }
-    // S^T: s[u][i] = key kb + 16u + 4grp + i, head column l16
-    df32x4_t s[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      s[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dbf16x8_t, kr[buf][u][0]),
-                                                     qb[0], df32x4_t{}, 0, 0, 0);
-      s[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dbf16x8_t, kr[buf][u][1]),
-                                                     qb[1], s[u], 0, 0, 0);
-    }
-    if (kb + TK > k_end) {
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (kb + 16 * u + 4 * grp + i >= k_end) s[u][i] = -INFINITY;
-    }
-    float mx = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
-                     fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float m_new = fmaxf(m, mx);
-    const float m_use = m_new == -INFINITY ? 0.f : m_new;
-    const float mc = m_use * c;
-    const float alpha = __builtin_amdgcn_exp2f(m * c - mc);
-    float rs = 0.f;
-    dbf16x8_t pb;
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float e = __builtin_amdgcn_exp2f(fmaf(s[u][i], c, -mc));
-        rs += e;
-        pb[4 * u + i] = (__bf16)e;  // k-slot (grp, 4u+i) = key 16u + 4grp + i
-      }
-    l = l * alpha + rs;  // this lane group's keys; groups are summed at the end
-    m = m_new;
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-      o[dt] *= alpha;
-      const bf16_t *row = vt + (16 * dt + l16) * VTP + 4 * grp;
-      const dbf16x4_t lo = *(const dbf16x4_t *)(row);       // keys 4grp .. +3
-      const dbf16x4_t hi = *(const dbf16x4_t *)(row + 16);  // keys 16 + 4grp .. +3
-      const dbf16x8_t a = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb, o[dt], 0, 0, 0);
-    }
-  };
-
-  // This wave's tiles: wave, wave+4, wave+8, ... (the workgroup walks the chunk
-  // front to back).  Every gload is unconditional, with the tile index clamped
-  // to the last tile (a repeated tile is an L2 hit): the same number of loads
-  // is then in flight on every path, and the compiler waits for one buffer
-  // only (vmcnt(8)) instead of draining both.
-  auto tile_kb = [&](int ti) { return k_begin + TK * min(ti, ntiles - 1); };
-#pragma unroll
-  for (int j = 0; j < NBUF; ++j) gload(j, tile_kb(wave + 4 * j));
-  for (int ti = wave; ti < ntiles; ti += 4 * NBUF) {
-#pragma unroll
-    for (int j = 0; j < NBUF; ++j) {
-      if (ti + 4 * j < ntiles) compute(j, k_begin + TK * (ti + 4 * j));
-      gload(j, tile_kb(ti + 4 * j + 4 * NBUF));
-    }
-  }
-
-  // o[dt][i] = O^T[d = 16dt + 4grp + i][head l16]; m is uniform over lane groups
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
-  float *red_o = reinterpret_cast<float *>(vt);  // [G][HD], this wave's V^T tile is done
-  if (l16 < G) {
-    if (grp == 0) {
-      red_m[wave][l16] = m;
-      red_l[wave][l16] = l;
-    }
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) red_o[l16 * HD + 16 * dt + 4 * grp + i] = o[dt][i];
-  }
-  __syncthreads();
-  for (int idx = tid; idx < G * HD; idx += 256) {
-    const int h = idx / HD, d = idx % HD;
-    float M = red_m[0][h];
-#pragma unroll
-    for (int w2 = 1; w2 < 4; ++w2) M = fmaxf(M, red_m[w2][h]);
-    const float Mu = M == -INFINITY ? 0.f : M;
-    float L = 0.f, A = 0.f;
-#pragma unroll
-    for (int w2 = 0; w2 < 4; ++w2) {
-      const float f = __builtin_amdgcn_exp2f((red_m[w2][h] - Mu) * c);
-      L += red_l[w2][h] * f;
-      A += reinterpret_cast<const float *>(Vt[w2])[h * HD + d] * f;
-    }
-    float *part = p.ws + (((int64_t)b * p.n_heads + g * G + h) * p.n_split + split) * (HD + 2);
-    part[2 + d] = A;
-    if (d == 0) {
-      part[0] = M * c;  // partials carry the max in the log2 domain
-      part[1] = L;
-    }
-  }
-}
-
-// bf16 cache, n_kv_heads a multiple of 4: whole-row streaming version.
-// A workgroup = (sequence, 4 consecutive KV heads, chunk).  Its 256 threads
-// load each 32-key tile as 16-byte chunks of the 4 heads' 128-byte key rows
-// (in a token-major cache one load instruction covers 1 KB: two token rows
-// of the 4 heads, which streams HBM far better than per-head 64-byte
-// pieces; other layouts reach each head's row through the head stride),
-// into registers two tiles ahead, then write it row-major to LDS.  Wave w is KV head g0 + w:
-// K fragments come from LDS with ds_read_b128, V^T fragments with the gfx950
-// transpose read ds_read_b64_tr_b16, and the wave writes its own partials.
 typedef short ds4_t __attribute__((ext_vector_type(4)));
-constexpr int RKP = 4 * HD + 8;   // K tile row pitch (elements): 528 B, 16 rows hit 64 distinct banks
-constexpr int RVP = 4 * HD + 16;  // V tile row pitch: 544 B, 4 rows x 32 B transpose reads conflict-free
-constexpr int RCH = TK * 4 * HD * 2 / 16 / 256;  // 16-byte chunks per thread per array per tile
-
 __device__ __forceinline__ dbf16x4_t lds_read_tr16(const bf16_t *p) {
   const ds4_t r = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
       (__attribute__((address_space(3))) ds4_t *)(__attribute__((address_space(3))) void *)p);
   return __builtin_bit_cast(dbf16x4_t, r);
-}
-
-template <int G>
-// register budget for 2 waves per SIMD (two register tiles ahead)
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void decode_bf16_rows_kernel(DecodeParams p) {
-  // two tile buffers: one barrier per tile orders the LDS writes and reads
-  __shared__ __attribute__((aligned(16))) bf16_t KL[2][TK * RKP];
-  __shared__ __attribute__((aligned(16))) bf16_t VL[2][TK * RVP];
-
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int l16 = lane & 15, grp = lane >> 4;
-  const int hblocks = p.n_kv_heads >> 2;
-  const int split = blockIdx.x % p.n_split;
-  const int bh = blockIdx.x / p.n_split;
-  const int b = bh / hblocks, g0 = (bh % hblocks) * 4;
-  const int g = g0 + wave;
-
-  int len = p.lens[b];
-  len = len < 0 ? 0 : (len > p.max_len ? p.max_len : len);
-  const int k_begin = split * p.chunk;
-  if (k_begin >= len) return;  // the combine kernel ignores chunks past len
-  const int k_end = min(k_begin + p.chunk, len);
-  const int ntiles = (k_end - k_begin + TK - 1) / TK;
-
-  const int64_t kv_rs = p.kv_rs;
-  const bf16_t *Kr = (const bf16_t *)p.k + b * p.kv_bs + g0 * p.kv_hs;
-  const bf16_t *Vr = (const bf16_t *)p.v + b * p.kv_bs + g0 * p.kv_hs;
-
-  dbf16x8_t qb[2];
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    if (l16 < G)
-      qb[t] = *(const dbf16x8_t *)((const bf16_t *)p.q +
-                                   ((int64_t)b * p.n_heads + g * G + l16) * HD + 8 * grp + 32 * t);
-    else
-      qb[t] = dbf16x8_t{};
-  }
-
-  // chunk c = tid + 256*i of a tile: row c / 32 (key), column (c % 32) * 8 elements.
-  // Two register tiles (A, B) hold the next two tiles' K and V chunks.
-  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));  // native vector: stays in VGPRs
-  struct RegTile {
-    u32x4 k0, k1, k2, k3, v0, v1, v2, v3;
-  };
-  static_assert(RCH == 4, "register tile holds 4 chunks per array");
-  const int crow = tid >> 5, ccol = (tid & 31) * 8;  // chunk i adds 8 rows
-  const int64_t cofs = (ccol >> 6) * p.kv_hs + (ccol & 63);  // head ccol/64 of the four
-  auto gload = [&](RegTile &r, int ti) __attribute__((always_inline)) {
-    const int kb = k_begin + TK * min(ti, ntiles - 1);  // clamped: same load count on every path
-    const int last = k_end - 1;  // past the end: a valid row, masked to P = 0
-    const int64_t o0 = (int64_t)min(kb + crow, last) * kv_rs + cofs;
-    const int64_t o1 = (int64_t)min(kb + crow + 8, last) * kv_rs + cofs;
-    const int64_t o2 = (int64_t)min(kb + crow + 16, last) * kv_rs + cofs;
-    const int64_t o3 = (int64_t)min(kb + crow + 24, last) * kv_rs + cofs;
-    // streamed once: non-temporal loads
-    r.k0 = __builtin_nontemporal_load((const u32x4 *)(Kr + o0)); r.v0 = __builtin_nontemporal_load((const u32x4 *)(Vr + o0));
-    r.k1 = __builtin_nontemporal_load((const u32x4 *)(Kr + o1)); r.v1 = __builtin_nontemporal_load((const u32x4 *)(Vr + o1));
-    r.k2 = __builtin_nontemporal_load((const u32x4 *)(Kr + o2)); r.v2 = __builtin_nontemporal_load((const u32x4 *)(Vr + o2));
-    r.k3 = __builtin_nontemporal_load((const u32x4 *)(Kr + o3)); r.v3 = __builtin_nontemporal_load((const u32x4 *)(Vr + o3));
-  };
-  auto lstore = [&](const RegTile &r, int buf) __attribute__((always_inline)) {
-    bf16_t *kd = KL[buf], *vd = VL[buf];
-    *(u32x4 *)(kd + crow * RKP + ccol) = r.k0;
-    *(u32x4 *)(kd + (crow + 8) * RKP + ccol) = r.k1;
-    *(u32x4 *)(kd + (crow + 16) * RKP + ccol) = r.k2;
-    *(u32x4 *)(kd + (crow + 24) * RKP + ccol) = r.k3;
-    *(u32x4 *)(vd + crow * RVP + ccol) = r.v0;
-    *(u32x4 *)(vd + (crow + 8) * RVP + ccol) = r.v1;
-    *(u32x4 *)(vd + (crow + 16) * RVP + ccol) = r.v2;
-    *(u32x4 *)(vd + (crow + 24) * RVP + ccol) = r.v3;
-  };
-  RegTile ta, tb;
-
-  float m = -INFINITY, l = 0.f;
-  df32x4_t o[4] = {df32x4_t{}, df32x4_t{}, df32x4_t{}, df32x4_t{}};
-  const float c = p.c;
-  auto compute = [&](int kb, int buf) __attribute__((always_inline)) {
-    const bf16_t *kl = KL[buf] + wave * HD + 8 * grp;  // this wave's head inside the tile
-    const bf16_t *vl = VL[buf] + wave * HD;
-    df32x4_t s[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const bf16_t *kp = kl + (16 * u + l16) * RKP;
-      s[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const dbf16x8_t *)(kp), qb[0], df32x4_t{},
-                                                     0, 0, 0);
-      s[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const dbf16x8_t *)(kp + 32), qb[1], s[u],
-                                                     0, 0, 0);
-    }
-    if (kb + TK > k_end) {
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (kb + 16 * u + 4 * grp + i >= k_end) s[u][i] = -INFINITY;
-    }
-    float mx = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
-                     fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float m_new = fmaxf(m, mx);
-    const float m_use = m_new == -INFINITY ? 0.f : m_new;
-    const float mc = m_use * c;
-    const float alpha = __builtin_amdgcn_exp2f(m * c - mc);
-    float rs = 0.f;
-    dbf16x8_t pb;
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float e = __builtin_amdgcn_exp2f(fmaf(s[u][i], c, -mc));
-        rs += e;
-        pb[4 * u + i] = (__bf16)e;  // k-slot (grp, 4u+i) = key 16u + 4grp + i
-      }
-    l = l * alpha + rs;
-    m = m_new;
-    // V^T operand: slot j of lane (grp, l16) = V[key 16(j/4) + 4grp + j%4][16dt + l16];
-    // transpose read: local lane n supplies V[key 4grp + n/4 (+16)][16dt + 4(n%4) .. +3]
-    const bf16_t *vp = vl + (4 * grp + (l16 >> 2)) * RVP + 4 * (l16 & 3);
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-      o[dt] *= alpha;
-      const dbf16x4_t lo = lds_read_tr16(vp + 16 * dt);
-      const dbf16x4_t hi = lds_read_tr16(vp + 16 * RVP + 16 * dt);
-      const dbf16x8_t a = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb, o[dt], 0, 0, 0);
-    }
-  };
-
-  // tile ti lives in LDS buffer ti & 1 and in register tile ta (even) / tb
-  // (odd), loaded two tiles ahead.  Writing buffer x for tile t happens after
-  // the barrier that follows the reads of tile t-2 (same buffer).
-  gload(ta, 0);
-  gload(tb, 1);
-  lstore(ta, 0);
-  gload(ta, 2);
-  __syncthreads();
-  for (int ti = 0; ti < ntiles; ti += 2) {
-    compute(k_begin + TK * ti, 0);
-    if (ti + 1 < ntiles) {  // workgroup-uniform
-      lstore(tb, 1);
-      gload(tb, ti + 3);
-      __syncthreads();
-      compute(k_begin + TK * (ti + 1), 1);
-      lstore(ta, 0);
-      gload(ta, ti + 4);
-      __syncthreads();
-    }
-  }
-
-  // o[dt][i] = O^T[d = 16dt + 4grp + i][query head g*G + l16]; m is uniform over lane groups
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
-  if (l16 < G) {
-    float *part = p.ws + (((int64_t)b * p.n_heads + g * G + l16) * p.n_split + split) * (HD + 2);
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) part[2 + 16 * dt + 4 * grp + i] = o[dt][i];
-    if (grp == 0) {
-      part[0] = m * c;  // log2 domain, as the other split kernels
-      part[1] = l;
-    }
-  }
 }
 
 // bf16 cache, one workgroup per (sequence, KV head) over the whole cache:
@@ -727,7 +375,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void d
 // streams them through a private LDS tile (no workgroup barrier in the loop):
 // 16-byte loads of the head's 128-byte cache rows, 8 rows per instruction,
 // the next tile register-staged; the scores and P V on
-// v_mfma_f32_16x16x32_bf16 as in the whole-row kernel.  The waves'
+// v_mfma_f32_16x16x32_bf16 as above.  The waves'
 // (m, l, acc) are merged through LDS at the end and the workgroup writes the
 // G output rows.  Four waves stream a cache (8 measured 8% slower on config
 // 3, 2 3% slower).  When a KV head's rows are contiguous (row stride
@@ -738,37 +386,73 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void d
 // keep four); token-major caches stream slower with more waves and keep four.
 constexpr int WWV = 4;  // streaming waves per workgroup
 constexpr int WWX = 6;  // waves of an adaptive whole-cache workgroup, active for a long cache
+constexpr int WW1 = 8;  // waves of the split kernel's unsplit pairs
 constexpr int kMeanBatchMax = 512;  // longer batches: four waves for every cache
 constexpr int WKP = HD + 8;  // tile row pitch, 144 B: b128 K reads of 16 rows and tr16 V
                              // reads of 4 rows x 32 B hit distinct banks
 
-// NW waves per workgroup: WWV, or WWX with the long-cache adaptation
-template <int G, int NW>
+// a cache up to this length is one split's (500 keys: 5.8 us, in 2-8 splits 6.9)
+constexpr int kSplitMinLen = 512;
+constexpr unsigned long long kArrive = 0x5bd1e995a93c71d4ull;
+// keys per split of a cache: whole rounds of the workgroup's four tiles
+template <int NW>
+__device__ __forceinline__ int split_chunk(int len, int n_split) {
+  if (len <= kSplitMinLen) return max(len, 1);
+  const int c = (len + n_split - 1) / n_split;
+  return max((c + NW * TK - 1) / (NW * TK), 1) * (NW * TK);
+}
+
+// NW waves per workgroup: WWV, or WWX with the long-cache adaptation.
+// SPLIT (fewer (sequence, KV head) pairs than compute units): n_split
+// workgroups per pair, each over a run of the cache, so that a few caches
+// have most of their loads in flight at once; bound by latencies (launch, one
+// or two memory round trips, the merge).  A split writes its merged (m, l,
+// acc) record through to memory, waits for it, and counts itself in on the
+// pair's arrival word; the last one to arrive merges the records and writes
+// the output, in the same launch.  Measured (graph replay, B=1 / 4 KV heads, G
+// 8) against the former chunk kernel over 4 KV heads' whole rows with its
+// combine launch: one cache of 1543 keys 9.9 -> 7.0 us, of 200 8.5 -> 4.5, of
+// 8000 18.0 -> 11.0; 12 caches of 200..4000 keys 16.9 -> 11.2, 32 of 500..2000
+// 17.5 -> 13.0, 48 of 500..4000 34.4 -> 25.2.
+// The arrival words stand at the workspace's end.  The first holds kArrive
+// between calls and counts up from it: one atomic.  Anything else there (a
+// fresh workspace) sends every split of the launch to the second word, where a
+// count starts under the launch's tag: a load and a compare-exchange that the
+// splits contend for (12 caches in 8 splits: 17.4 against 12.2 us).  The last
+// arrival leaves kArrive, so neither a fresh workspace nor a replayed graph
+// needs a clearing pass.
+template <int G, int NW, bool SPLIT>
 __global__ __launch_bounds__(64 * NW) void decode_bf16_whole_kernel(DecodeParams p) {
   __shared__ __attribute__((aligned(16))) bf16_t KT[NW][TK * WKP];
   __shared__ __attribute__((aligned(16))) bf16_t VT[NW][TK * WKP];
   __shared__ float red_m[NW][G], red_l[NW][G];
   __shared__ float red_o[NW][G][HD];
+  __shared__ int last_split;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, grp = lane >> 4;
-  const int b = blockIdx.x / p.n_kv_heads, g = blockIdx.x % p.n_kv_heads;
+  // the KV heads of a sequence's (split's) rows next to each other
+  const int g = blockIdx.x % p.n_kv_heads, bs = blockIdx.x / p.n_kv_heads;
+  const int b = SPLIT ? bs / p.n_split : bs, split = SPLIT ? bs - b * p.n_split : 0;
   auto clamp_len = [&](int x) { return x < 0 ? 0 : (x > p.max_len ? p.max_len : x); };
 
   // the batch's total length (batches up to kMeanBatchMax sequences), summed
   // by every wave itself (no barrier), read with this sequence's length
-  const bool adapt = NW > WWV && p.batch <= kMeanBatchMax;
+  const bool adapt = !SPLIT && NW > WWV && p.batch <= kMeanBatchMax;
   int part = 0;
   if (adapt)
     for (int i = lane; i < p.batch; i += 64) part += clamp_len(p.lens[i]);
   const int len = clamp_len(p.lens[b]);
   bf16_t *out = (bf16_t *)p.o + ((int64_t)b * p.n_heads + (int64_t)g * G) * HD;
+  const int chunk = SPLIT ? split_chunk<NW>(len, p.n_split) : 0;
+  const int k0 = split * chunk;
+  if (SPLIT && split > 0 && k0 >= len) return;
   if (len == 0) {  // no key: zeros
     for (int idx = tid; idx < G * HD; idx += 64 * NW) out[idx] = f32_to_bf16(0.f);
     return;
   }
-  int nw = WWV;  // streaming waves of this workgroup (uniform)
+  int nw = SPLIT ? NW : WWV;  // streaming waves of this workgroup (uniform)
   if (adapt) {
 #pragma unroll
     for (int o2 = 32; o2 > 0; o2 >>= 1) part += __shfl_xor(part, o2, 64);
@@ -778,8 +462,9 @@ __global__ __launch_bounds__(64 * NW) void decode_bf16_whole_kernel(DecodeParams
   // wave w < nw takes the 32-key tiles w, w + nw, w + 2*nw, ...: the waves of
   // a workgroup stream adjacent tiles (a contiguous key range per wave, or the
   // KV heads of one sequence placed on one XCD, measured 3-4% slower)
-  const int all_tiles = (len + TK - 1) / TK;
-  const int kw0 = TK * wave, kw1 = len;
+  const int kw1 = SPLIT ? min(k0 + chunk, len) : len;
+  const int all_tiles = (kw1 - k0 + TK - 1) / TK;
+  const int kw0 = k0 + TK * wave;
   const int tstride = TK * nw;  // keys between a wave's tiles
   const int ntiles = wave < nw && all_tiles > wave ? (all_tiles - wave + nw - 1) / nw : 0;
 
@@ -921,6 +606,7 @@ __global__ __launch_bounds__(64 * NW) void decode_bf16_whole_kernel(DecodeParams
     }
   }
   __syncthreads();
+  const int nvalid = SPLIT ? (len + chunk - 1) / chunk : 1;  // splits that hold keys
   for (int idx = tid; idx < G * HD; idx += 64 * NW) {
     const int h = idx / HD, d = idx - h * HD;
     float M = red_m[0][h];
@@ -933,7 +619,54 @@ __global__ __launch_bounds__(64 * NW) void decode_bf16_whole_kernel(DecodeParams
       L += red_l[w][h] * wt;
       A += red_o[w][h][d] * wt;
     }
-    out[idx] = f32_to_bf16(A / L);
+    if (!SPLIT || nvalid == 1) {
+      out[idx] = f32_to_bf16(A / L);
+    } else {
+      float *rec = p.ws + (((int64_t)b * p.n_heads + (int64_t)g * G + h) * p.n_split + split) * kDecRec;
+      auto wr = [](float *q, float v) { __hip_atomic_store(q, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); };
+      wr(rec + 2 + d, A);
+      if (d == 0) {
+        wr(rec, M);
+        wr(rec + 1, L);
+      }
+    }
+  }
+  if constexpr (SPLIT) {
+    if (nvalid == 1) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the record's stores have reached memory
+    __syncthreads();
+    if (tid == 0) {
+      unsigned long long *word = p.arrive_end - 2 * ((int64_t)b * p.n_kv_heads + g + 1);
+      unsigned long long old = __hip_atomic_fetch_add(word, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      bool last = old - kArrive == (unsigned long long)(nvalid - 1);
+      if (old - kArrive >= (unsigned long long)nvalid) {
+        unsigned long long next;
+        old = __hip_atomic_load(word + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        do {
+          next = (old >> 16 == p.tag ? old : p.tag << 16) + 1;
+        } while (!__hip_atomic_compare_exchange_strong(word + 1, &old, next, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                       __HIP_MEMORY_SCOPE_AGENT));
+        last = (int)(next & 0xffff) == nvalid;
+      }
+      if (last) __hip_atomic_store(word, kArrive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      last_split = last;
+    }
+    __syncthreads();
+    if (!last_split) return;
+    for (int idx = tid; idx < G * (HD / 4); idx += 64 * NW) {
+      const int h = idx / (HD / 4), d0 = 4 * (idx % (HD / 4));
+      const float *rec = p.ws + ((int64_t)b * p.n_heads + (int64_t)g * G + h) * p.n_split * kDecRec;
+      DecMerge mg;
+      mg.start();
+      for (int s0 = 0; s0 < nvalid; s0 += 8) {
+        mg.load8<true>(rec, p.n_split, s0, d0);
+        mg.merge8(s0, nvalid);
+      }
+      const float4 r = mg.result();
+      const uint32_t lo = (uint32_t)f32_to_bf16(r.x) | ((uint32_t)f32_to_bf16(r.y) << 16);
+      const uint32_t hi = (uint32_t)f32_to_bf16(r.z) | ((uint32_t)f32_to_bf16(r.w) << 16);
+      *(uint2 *)(out + h * HD + d0) = make_uint2(lo, hi);
+    }
   }
 }
 
@@ -1451,8 +1184,8 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(DecodeParams p) {
   Elem<T>::store(out + 3, r.w);
 }
 
-// split-K workgroup targets: per-head kernels / whole-row kernel (4 KV heads
-// per workgroup)
+// workgroup targets of the fp32 chunks, and of the four-KV-head bf16 chunks
+// that the no-allocation call's size limit is stated in
 constexpr int kMinWg = 2048, kRowsMinWg = 512;
 int choose_chunk(int batch, int max_len, int units, int min_wg) {
   // enough workgroups to cover the 256 CUs several times over (a partial last
@@ -1463,21 +1196,7 @@ int choose_chunk(int batch, int max_len, int units, int min_wg) {
   return chunk;
 }
 
-template <typename T, int G>
-void launch_split(const DecodeParams &p, dim3 grid, hipStream_t s) {
-  if constexpr (std::is_same<T, bf16_t>::value) {
-    if (p.n_kv_heads % 4 == 0)
-      hipLaunchKernelGGL((decode_bf16_rows_kernel<G>), grid, dim3(256), 0, s, p);
-    else
-      hipLaunchKernelGGL((decode_bf16_mfma_kernel<G>), grid, dim3(256), 0, s, p);
-  } else {
-    hipLaunchKernelGGL((decode_split_kernel<T, G, 4, DEC_SPLIT>), grid, dim3(256), 0, s, p);
-  }
-}
-
 bool rows_path(const DecodeParams &p, bool bf16) { return bf16 && p.n_kv_heads % 4 == 0; }
-
-
 
 void launch_short(const DecodeParams &p, hipStream_t s) {
   const dim3 grid((unsigned)((int64_t)p.batch * p.n_heads / kShortG * p.n_split));
@@ -1485,22 +1204,18 @@ void launch_short(const DecodeParams &p, hipStream_t s) {
                      0, s, p);
 }
 
-template <typename T>
+// fp32 caches past the short split: chunks, then the combine
 int launch_decode(const DecodeParams &p, int G, hipStream_t s) {
-  const bool rows = rows_path(p, std::is_same<T, bf16_t>::value);
-  const dim3 grid((unsigned)((int64_t)p.batch * (rows ? p.n_kv_heads / 4 : p.n_kv_heads) *
-                             p.n_split));
+  const dim3 grid((unsigned)((int64_t)p.batch * p.n_kv_heads * p.n_split));
   switch (G) {
-    case 0: launch_short(p, s); break;  // short-cache split (fp32)
-    case 1: launch_split<T, 1>(p, grid, s); break;
-    case 2: launch_split<T, 2>(p, grid, s); break;
-    case 4: launch_split<T, 4>(p, grid, s); break;
-    default: launch_split<T, 8>(p, grid, s); break;
+    case 1: hipLaunchKernelGGL((decode_split_kernel<float, 1, 4, DEC_SPLIT>), grid, dim3(256), 0, s, p); break;
+    case 2: hipLaunchKernelGGL((decode_split_kernel<float, 2, 4, DEC_SPLIT>), grid, dim3(256), 0, s, p); break;
+    case 4: hipLaunchKernelGGL((decode_split_kernel<float, 4, 4, DEC_SPLIT>), grid, dim3(256), 0, s, p); break;
+    default: hipLaunchKernelGGL((decode_split_kernel<float, 8, 4, DEC_SPLIT>), grid, dim3(256), 0, s, p);
   }
   BN_LAUNCH_CHECK();
   const int64_t n = (int64_t)p.batch * p.n_heads * (HD / 4);
-  hipLaunchKernelGGL(decode_combine_kernel<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-                     s, p);
+  hipLaunchKernelGGL(decode_combine_kernel<float>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p);
   BN_LAUNCH_CHECK();
   return BN_OK;
 }
@@ -1572,6 +1287,27 @@ uint32_t next_plan_epoch() {
   uint32_t e = g_plan_epoch.fetch_add(1) + 1;
   if (e == 0) e = g_plan_epoch.fetch_add(1) + 1;
   return e;
+}
+// Splits per (sequence, KV head) pair of the split whole-cache kernel: about
+// one workgroup per compute unit, at most 8 records to merge (us, by splits:
+// one cache of 1543 keys 1 / 4 / 8 / 12 11.2 / 8.1 / 7.0 / 7.1; 12 caches of
+// 200..4000 4 / 5 / 8 12.4 / 11.2 / 12.0; 16 of 4000, 4 KV heads, 2 / 4 / 8
+// 19.3 / 13.9 / 16.7; 32 of 500..2000 1 / 2 / 4 16.1 / 13.0 / 15.0; 48 of
+// 500..4000 1 / 2 28.4 / 28.8), and one fewer than the cache's 128-key chunks,
+// so that the records and the arrival words fit the workspace that
+// bn_gqa_decode_workspace_size() asks for.  Unsplit pairs have eight waves
+// (48 caches: 28.4 -> 25.2; 60 of 100..1000 11.6 -> 11.0), split ones four.
+int whole_splits(int units, int max_len) {
+  return std::max(1, std::min({256 / units, 8, (max_len + 127) / 128 - 1}));
+}
+// a launch's 48-bit tag: a mixed counter (SplitMix64's finaliser), so that
+// no plausible memory contents look like this launch's arrivals
+std::atomic<uint64_t> g_split_launch{0};
+unsigned long long next_split_tag() {
+  uint64_t z = (g_split_launch.fetch_add(1) + 1) * 0x9e3779b97f4a7c15ull;
+  z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
+  z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
+  return (z ^ (z >> 31)) >> 16 | 1;
 }
 // the next counter slot of the short-cache decode on `device` (null: not set up)
 constexpr int kShortSlots = 16;
@@ -1675,9 +1411,9 @@ int gqa_decode_impl(int dtype, const void *q, const void *k_cache, const void *v
 #define BN_WHOLE(GG)                                                                        \
   do {                                                                                      \
     if (wide)                                                                               \
-      hipLaunchKernelGGL((decode_bf16_whole_kernel<GG, WWX>), grid, block, 0, s, p);        \
+      hipLaunchKernelGGL((decode_bf16_whole_kernel<GG, WWX, false>), grid, block, 0, s, p);        \
     else                                                                                    \
-      hipLaunchKernelGGL((decode_bf16_whole_kernel<GG, WWV>), grid, block, 0, s, p);        \
+      hipLaunchKernelGGL((decode_bf16_whole_kernel<GG, WWV, false>), grid, block, 0, s, p);        \
   } while (0)
       switch (G) {
         case 1: BN_WHOLE(1); break;
@@ -1694,19 +1430,25 @@ int gqa_decode_impl(int dtype, const void *q, const void *k_cache, const void *v
     p.chunk = 0;
     p.n_split = kShortSplits;
   } else {
-    // the whole-row kernel gives each workgroup 4 KV heads: 1/4 of the workgroups per chunk
     p.chunk = rows_path(p, dtype == BN_BF16)
                   ? choose_chunk(batch, max_len, n_kv_heads / 4, kRowsMinWg)
                   : choose_chunk(batch, max_len, n_kv_heads, kMinWg);
     p.n_split = (max_len + p.chunk - 1) / p.chunk;
   }
   p.c = scale * 1.4426950408889634f;
-  const size_t need = (size_t)batch * n_heads * p.n_split * (HD + 2) * sizeof(float);
+  const bool bsplit = !short_split && dtype == BN_BF16;  // split whole-cache kernel
+  size_t need = (size_t)batch * n_heads * p.n_split * (HD + 2) * sizeof(float);
   if (noalloc && need > (size_t)BN_GQA_DECODE_SCRATCH_BYTES)
     return fail(BN_ERR_UNSUPPORTED, std::string(op) + ": the call needs " + std::to_string(need) +
                                         " bytes of chunk partials, above the " +
                                         std::to_string((size_t)BN_GQA_DECODE_SCRATCH_BYTES) +
                                         "-byte scratch");
+  size_t words = 0;
+  if (bsplit) {  // (the no-allocation limit above stays that of the chunks' partials)
+    p.n_split = whole_splits(batch * n_kv_heads, max_len);
+    words = p.n_split > 1 ? (size_t)batch * n_kv_heads * 16 + 8 : 0;
+    need = p.n_split > 1 ? (size_t)batch * n_heads * p.n_split * kDecRec * sizeof(float) + words : 0;
+  }
   int st = ensure_device();
   if (st) return st;
   hipStream_t s = as_stream(stream);
@@ -1718,12 +1460,35 @@ int gqa_decode_impl(int dtype, const void *q, const void *k_cache, const void *v
     ws = decode_scratch(library_device());
     if (!ws) return fail(BN_ERR_HIP, std::string(op) + ": scratch address not set up for device " +
                                          std::to_string(library_device()));
-  } else if (!ws) {
+  } else if (!ws && need > 0) {
     if ((st = bn_alloc(&ws, need, stream))) return st;
     own = true;
   }
   p.ws = (float *)ws;
-  if (short_split) {  // one launch: the unit's last split merges its records
+  if (bsplit) {  // one launch: a pair's last split merges its records
+    if (words) {
+      const size_t bytes = noalloc ? (size_t)BN_GQA_DECODE_SCRATCH_BYTES : own ? need : workspace_bytes;
+      p.arrive_end = (unsigned long long *)(((uintptr_t)ws + bytes) & ~(uintptr_t)7);
+      p.tag = next_split_tag();
+    }
+    const dim3 grid((unsigned)((int64_t)batch * n_kv_heads * p.n_split));
+#define BN_SPLIT(GG)                                                                                  \
+  do {                                                                                                \
+    if (p.n_split > 1)                                                                                \
+      hipLaunchKernelGGL((decode_bf16_whole_kernel<GG, WWV, true>), grid, dim3(64 * WWV), 0, s, p);   \
+    else                                                                                              \
+      hipLaunchKernelGGL((decode_bf16_whole_kernel<GG, WW1, true>), grid, dim3(64 * WW1), 0, s, p);   \
+  } while (0)
+    switch (G) {
+      case 1: BN_SPLIT(1); break;
+      case 2: BN_SPLIT(2); break;
+      case 4: BN_SPLIT(4); break;
+      default: BN_SPLIT(8); break;
+    }
+#undef BN_SPLIT
+    const hipError_t e = hipGetLastError();
+    st = e == hipSuccess ? BN_OK : hip_fail(e, __FILE__, __LINE__);
+  } else if (short_split) {  // one launch: the unit's last split merges its records
     p.cnt = short_counter_slot(library_device());
     if (!p.cnt) {
       st = fail(BN_ERR_HIP, std::string(op) + ": split counters not set up for device " +
@@ -1734,7 +1499,7 @@ int gqa_decode_impl(int dtype, const void *q, const void *k_cache, const void *v
       st = e == hipSuccess ? BN_OK : hip_fail(e, __FILE__, __LINE__);
     }
   } else {
-    st = dtype == BN_BF16 ? launch_decode<bf16_t>(p, G, s) : launch_decode<float>(p, G, s);
+    st = launch_decode(p, G, s);
   }
   if (own) {
     int st2 = bn_free(ws, stream);

@@ -337,7 +337,11 @@ int bn_llama_decode(const bn_llama_config *config, const float *embed,
  * whole cache is attended).  workspace: device memory of
  * bn_gqa_decode_workspace_size() bytes (NULL: taken from the pool when the
  * call needs it); single-pass calls use none: bf16 caches with
- * batch*n_kv_heads >= the device's compute units.  fp32 caches of at most
+ * batch*n_kv_heads above half the device's compute units or of at most 256
+ * keys.  Other bf16 calls keep split records there and, at its end, arrival
+ * words that the splits count in on; a call whose workspace the previous call
+ * also used (any shape) finds them ready, and on any other contents the count
+ * takes a slower path to the same result.  fp32 caches of at most
  * 1024 keys with batch*n_heads <= 256 keep 4 split records per (sequence,
  * head) in it and merge them in the same launch, counting on a ring of 16
  * counter slots inside the library: at most 16 such calls in flight at once

@@ -703,3 +703,55 @@ def test_prefill_f32_wide_kv_rows():
 
     o = B.gqa_prefill(dev(q), wide(k, 0), wide(v, Hkv * 64), scale=0.125, seq_offset=2)
     assert_close(host(o), O.gqa_prefill(q, k, v, 0.125, True, 2), TOL["f32"])
+
+
+# the split whole-cache kernel (bf16, fewer (sequence, KV head) pairs than compute units): 1-8 splits, cache
+# lengths on both sides of a split's limits, group sizes, KV head counts that are no multiple of 4
+SPLIT_DECODE_CASES = [
+    # lengths, max_len, H, Hkv, head-major
+    ([1543], 2048, 32, 4, True),
+    ([512, 513, 0, 1, 1024, 1025], 1100, 8, 2, False),
+    ([4000, 127, 129, 640, 2049], 4096, 6, 3, False),
+    ([200], 256, 8, 8, True),                # one split: no workspace used
+    ([700, 1300, 385], 1300, 4, 4, True),
+    ([900] * 33, 1000, 8, 4, False),         # 132 pairs: unsplit, eight waves
+]
+
+
+@pytest.mark.parametrize("case", SPLIT_DECODE_CASES)
+def test_decode_bf16_split_in_one_launch(case):
+    lens, Lmax, H, Hkv, head_major = case
+    Bn = len(lens)
+    k, v = (draw((Bn, Lmax, Hkv, 64), 31 + i, "bf16") for i in range(2))
+
+    def cache(x):
+        t = dev(x, torch.bfloat16)
+        return t.transpose(1, 2).contiguous().transpose(1, 2) if head_major else t
+
+    kd, vd = cache(k), cache(v)
+    ld = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    ws = B.decode_workspace(Bn, Lmax, H)
+    ws.random_(0, 256)  # any contents: the first call's arrivals start under its tag
+    qd = torch.empty((Bn, H, 64), dtype=torch.bfloat16, device="cuda")
+    o = torch.empty_like(qd)
+
+    def check(seed, what):
+        q = draw((Bn, H, 64), seed, "bf16")
+        qd.copy_(dev(q, torch.bfloat16))
+        yield
+        ref = O.gqa_decode(q, k, v, np.array(lens, np.int32), 0.125)
+        assert_close(host(o), ref, BF16_TOL, f"{what} {case}")
+
+    def run(workspace=ws):
+        B.gqa_decode(qd, kd, vd, ld, o, scale=0.125, workspace=workspace)
+
+    for n, workspace in enumerate((ws, ws, None)):
+        for _ in check(40 + n, f"call {n}"):
+            run(workspace)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run()
+    for n in range(4):  # replays of one tag, an eager call of another between them
+        for _ in check(50 + n, f"replay {n}"):
+            graph.replay()
+        run()
