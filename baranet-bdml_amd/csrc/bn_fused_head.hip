@@ -1,4 +1,4 @@
-// bn_fused_head.hip -- the reference's fused-head attention chain in one launch.
+// bn_fused_head.hip -- the reference's fused-head attention chain in one launch or two.
 //
 // Replaces the chain of llama_layers.hpp:83-109 (fp32):
 //   K_rep = repeat_kv(K), V_rep = repeat_kv(V)       (:87-89, :131-168)
@@ -15,8 +15,9 @@
 // so the n_rep heads of a group receive the same values.  Neither K_rep,
 // V_rep nor the Sq x Sk matrices exist here.
 //
-// Work decomposition: a 256-thread workgroup (4 waves) owns R = 4 query rows
-// and walks the visible keys in tiles of 64 with an online softmax:
+// Short key ranges and widths other than 256 (the rest: the matrix-core path
+// below): a 256-thread workgroup (4 waves) owns R = 4 query rows and walks the
+// visible keys in tiles of 64 with an online softmax:
 //   1. the rows' Qsum (R x KV*D) is formed once into LDS;
 //   2. scores: thread (wave w, lane l) forms the R partial dots of key l over
 //      the w-th quarter of the contraction (each K element is loaded once per
@@ -284,37 +285,41 @@ __global__ __launch_bounds__(256) void fused_head_attention_kernel(FusedHeadPara
 }
 
 // ------------------------------------------------------- matrix-core path
-// Longer prompts (seq_q >= kMfmaMinRows) with KV*D = 256 (TinyLLaMA's 4 KV
-// heads of 64) run the same chain on v_mfma_f32_32x32x2f32, in three
-// launches:
-//   1. fh_qsum_kernel: Qs[i][c] = c2 * sum_{r < n_rep} Q_{g*n_rep + r}[i][d]
-//      (c = g*D + d, summed in r order; c2 = scale * log2 e, so the scores
-//      come out in log2 units), [seq_q, 256] in the workspace.
-//   2. fh_mfma_kernel: one workgroup per block of 32 query rows x 128 keys.
-//      Wave w forms S^T = K.Qs^T of the block's four 32-key tiles over its
-//      quarter (64 columns) of the contraction; the four quarters meet in LDS
-//      and are summed in wave order, so every wave holds the same 128 x 32
-//      scores.  Each wave masks them, takes the block's row max m, forms
-//      P = exp2(s - m) and l = sum P, and O[:, 64w .. 64w+63] = P.V for its
-//      quarter of the value columns (P straight from the score registers as
-//      the B operand).  The block writes its record (m, l, O[32][256]).
-//   3. fh_merge_kernel: each query row merges the records of its row tile
-//      (max of m, exp2-weighted sums of l and O), normalises, and writes the
-//      values of KV head g to the row's n_rep heads of group g.
-// Per block a wave runs 128 MFMAs for S and 128 for P.V; the blocks of a
-// prompt spread over every compute unit, where the VALU kernel's longest
-// rows walk every key tile on one compute unit each.
-constexpr int kMfmaMinRows = 512;  // shorter prompts: the VALU kernel (faster at 256 rows)
-constexpr int FH_KVD = 256, FH_ROWS = 32, FH_KEYS = 128;
-constexpr int FH_REC = 2 * FH_ROWS + FH_ROWS * FH_KVD;  // m[32], l[32], O[32][256]
+// KV*D = 256 (TinyLLaMA's 4 KV heads of 64) on v_mfma_f32_16x16x4f32, one
+// launch or two:
+//   1. fh_rows_kernel: a workgroup of 8 waves takes 16 query rows and one split
+//      of their visible keys.  The rows' group sums Qsum (times c2 = scale *
+//      log2 e: scores in log2 units; summed in head order) go to LDS once.  Each
+//      wave then walks its own 16-key tiles with an online softmax: S^T = K.Qs^T
+//      over the whole contraction (64 MFMAs in four chains), P straight from the
+//      score registers as the B operand of O^T += V^T.P^T (64 MFMAs, all 256
+//      value columns).  K and V go from memory to registers, no barrier in the
+//      loop; the waves meet in LDS once at the end.
+//   2. fh_merge_kernel, with more than one split: merges the splits' records.
+// What bounds it: at 512 rows nothing but latency (13.6 us: launch, Q, K and V
+// one after the other, 3.4 us of MFMAs, the merge of 8 waves; + 4.9 us for the
+// second launch); at 2048 rows and more the matrix rate (8256 tiles of 4096
+// cycles on 1024 SIMDs: 14 us of 50) and K/V from L2 (32 KB per tile).
+// Measured against one 32-row x 128-key block per workgroup with the group sums
+// and the merge in launches of their own and an allocation for both, us per
+// call: 512 rows 30-36 -> 18.1, 1024 rows 32-36 -> 27.3, 2048 rows 71.7 -> 50,
+// 8192 rows 696 -> 350, 512 rows + 1000 past 36 -> 27.6; and against the VALU
+// kernel at fewer rows: 200 rows 19.1 -> 13.2, 384 rows 27.1 -> 15.0, 64 rows +
+// 1000 past 65 -> 20.  V's first tile fetched before the barrier: 2-10% slower
+// (it delays K).
+constexpr int FH_KVD = 256, FH_ROWS = 16, FH_TILE = 16, FH_WAVES = 8, FH_SPLITS = 7;
 
-typedef float fh_f32x16 __attribute__((ext_vector_type(16)));
+typedef float fh_f32x4 __attribute__((ext_vector_type(4)));
 
 struct FhParams {
   const float *q, *k, *v;
-  float *o, *qs, *part;
-  int64_t ldq, ldk, ldv, ldo;
-  int sq, sk, n_heads, head_dim, n_rep, n_kc, causal, seq_offset;
+  float *o, *rec;                   // rec: the splits' records, one row per query row
+  int64_t ldq, ldk, ldv, ldo, ldr;  // row strides in elements
+  int sq, sk, head_dim, n_rep;
+  int n_split, ml;  // records per row; first column of a row's (m, l) pairs
+  int direct;       // one split: the workgroup writes the output itself
+  int nan_rows;     // a row whose sum is NaN: 1 gives NaN, 0 zeros
+  int causal, seq_offset;
   float c2;  // scale * log2(e)
 };
 
@@ -325,197 +330,311 @@ __device__ __forceinline__ int fh_key_end(const FhParams &p, int row) {
   return (int)(e < 0 ? 0 : (e > p.sk ? p.sk : e));
 }
 
-__global__ __launch_bounds__(256) void fh_qsum_kernel(FhParams p) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (int64_t)p.sq * (FH_KVD / 4)) return;
-  const int row = (int)(idx / (FH_KVD / 4)), c = (int)(idx % (FH_KVD / 4)) * 4;
-  const int g = c / p.head_dim, d = c - g * p.head_dim;
-  const float *qr = p.q + (int64_t)row * p.ldq + (int64_t)g * p.n_rep * p.head_dim + d;
-  float4 a = ld4(qr);
-  for (int r = 1; r < p.n_rep; ++r) {
-    const float4 b = ld4(qr + (int64_t)r * p.head_dim);
-    a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
-  }
-  *reinterpret_cast<float4 *>(p.qs + (int64_t)row * FH_KVD + c) =
-      make_float4(a.x * p.c2, a.y * p.c2, a.z * p.c2, a.w * p.c2);
+// keys per split of the row block that ends with key `kend`: whole tiles,
+// every row block's own tiles dealt evenly
+__device__ __forceinline__ int fh_chunk(const FhParams &p, int kend) {
+  const int tiles = (kend + FH_TILE - 1) / FH_TILE;
+  return (tiles + p.n_split - 1) / p.n_split * FH_TILE;
 }
 
-__global__ __launch_bounds__(256, 2) void fh_mfma_kernel(FhParams p) {
-  // the four waves' partial scores: [wave][key tile][register group][lane]
-  __shared__ float4 sbuf[4][4][4][64];
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  const int r32 = lane & 31, hf = lane >> 5;
-  const int kc = blockIdx.x % p.n_kc, rt = blockIdx.x / p.n_kc;
-  const int row0 = rt * FH_ROWS, key0 = kc * FH_KEYS;
-  const int kend_tile = fh_key_end(p, min(row0 + FH_ROWS - 1, p.sq - 1));
-  if (key0 >= kend_tile) return;  // no record: the merge counts the blocks the same way
-
-  // B operand of S^T: query row0 + r32, contraction slot (4u + e, hf) =
-  // column 64w + 8u + 4hf + e of Qs (rows past seq_q: zeros)
-  const int qrow = row0 + r32;
-  float qreg[32];
-#pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    const float4 a = qrow < p.sq ? ld4(p.qs + (int64_t)qrow * FH_KVD + 64 * w + 8 * u + 4 * hf) : zero4();
-    qreg[4 * u] = a.x; qreg[4 * u + 1] = a.y; qreg[4 * u + 2] = a.z; qreg[4 * u + 3] = a.w;
-  }
-  // A operand: key key0 + 32kt + r32 (clamped into the cache; masked below),
-  // the same contraction columns
-  auto load_k = [&](int kt, float4 (&kr)[8]) __attribute__((always_inline)) {
-    const int key = min(key0 + 32 * kt + r32, p.sk - 1);
-    const float *kp = p.k + (int64_t)key * p.ldk + 64 * w + 4 * hf;
-#pragma unroll
-    for (int u = 0; u < 8; ++u) kr[u] = ld4(kp + 8 * u);
-  };
-  fh_f32x16 s[4];
-#pragma unroll
-  for (int kt = 0; kt < 4; ++kt) {
-    float4 cur[8];
-    load_k(kt, cur);
-    s[kt] = fh_f32x16{};
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      s[kt] = __builtin_amdgcn_mfma_f32_32x32x2f32(cur[u].x, qreg[4 * u], s[kt], 0, 0, 0);
-      s[kt] = __builtin_amdgcn_mfma_f32_32x32x2f32(cur[u].y, qreg[4 * u + 1], s[kt], 0, 0, 0);
-      s[kt] = __builtin_amdgcn_mfma_f32_32x32x2f32(cur[u].z, qreg[4 * u + 2], s[kt], 0, 0, 0);
-      s[kt] = __builtin_amdgcn_mfma_f32_32x32x2f32(cur[u].w, qreg[4 * u + 3], s[kt], 0, 0, 0);
-    }
-  }
-  // the quarters of the contraction meet in LDS, summed in wave order
-#pragma unroll
-  for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-      sbuf[w][kt][g][lane] = make_float4(s[kt][4 * g], s[kt][4 * g + 1], s[kt][4 * g + 2], s[kt][4 * g + 3]);
-  __syncthreads();
-#pragma unroll
-  for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      float4 a = sbuf[0][kt][g][lane];
-#pragma unroll
-      for (int w2 = 1; w2 < 4; ++w2) {
-        const float4 b = sbuf[w2][kt][g][lane];
-        a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
-      }
-      s[kt][4 * g] = a.x; s[kt][4 * g + 1] = a.y; s[kt][4 * g + 2] = a.z; s[kt][4 * g + 3] = a.w;
-    }
-
-  // mask, row max, P = exp2(s - m), row sum; register i of s[kt] is key
-  // key0 + 32kt + 8(i/4) + 4hf + i%4 of query qrow
-  const int kend_row = qrow < p.sq ? fh_key_end(p, qrow) : 0;
-  float mx = -INFINITY;
-#pragma unroll
-  for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int key = key0 + 32 * kt + 8 * (i >> 2) + 4 * hf + (i & 3);
-      const float v = key < kend_row ? s[kt][i] : -INFINITY;
-      s[kt][i] = v;
-      mx = fmaxf(mx, v);
-    }
-  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-  const float mu = mx == -INFINITY ? 0.f : mx;
-  float l = 0.f;
-#pragma unroll
-  for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float e = __builtin_amdgcn_exp2f(s[kt][i] - mu);
-      s[kt][i] = e;
-      l += e;
-    }
-  l += __shfl_xor(l, 32, 64);
-
-  // O^T[value column][query] += V^T P^T over the block's keys: A = V^T (lane:
-  // column slot r32 of tile dt = value column 64w + 2*r32 + dt, key of the
-  // step's half hf), B = P^T (the score registers)
-  fh_f32x16 o[2] = {fh_f32x16{}, fh_f32x16{}};
-  auto load_v = [&](int kt, float2 (&vr)[16]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int key = min(key0 + 32 * kt + 8 * g + 4 * hf + e, p.sk - 1);
-        vr[4 * g + e] = *reinterpret_cast<const float2 *>(p.v + (int64_t)key * p.ldv + 64 * w + 2 * r32);
-      }
-  };
-#pragma unroll
-  for (int kt = 0; kt < 4; ++kt) {
-    float2 cur[16];
-    load_v(kt, cur);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      o[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(cur[i].x, s[kt][i], o[0], 0, 0, 0);
-      o[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(cur[i].y, s[kt][i], o[1], 0, 0, 0);
-    }
-  }
-
-  // the block's record: m and l per query (wave 0), O[query][column]:
-  // register i of o[dt] is column 64w + 2*(8(i/4) + 4hf + i%4) + dt of query qrow
-  float *rec = p.part + (int64_t)blockIdx.x * FH_REC;
-  if (w == 0 && hf == 0) {
-    rec[r32] = mx;
-    rec[FH_ROWS + r32] = l;
-  }
-  float *orow = rec + 2 * FH_ROWS + r32 * FH_KVD + 64 * w;
-#pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    const int c0 = 2 * (8 * g + 4 * hf);
-    *reinterpret_cast<float4 *>(orow + c0) = make_float4(o[0][4 * g], o[1][4 * g], o[0][4 * g + 1], o[1][4 * g + 1]);
-    *reinterpret_cast<float4 *>(orow + c0 + 4) =
-        make_float4(o[0][4 * g + 2], o[1][4 * g + 2], o[0][4 * g + 3], o[1][4 * g + 3]);
-  }
-}
-
-__global__ __launch_bounds__(256) void fh_merge_kernel(FhParams p) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (int64_t)p.sq * (FH_KVD / 4)) return;
-  const int row = (int)(idx / (FH_KVD / 4)), c = (int)(idx % (FH_KVD / 4)) * 4;
-  const int rt = row / FH_ROWS, r = row % FH_ROWS;
-  const int kend_tile = fh_key_end(p, min(rt * FH_ROWS + FH_ROWS - 1, p.sq - 1));
-  const int nblk = (kend_tile + FH_KEYS - 1) / FH_KEYS;  // the blocks that wrote a record
-  const float *rec0 = p.part + (int64_t)rt * p.n_kc * FH_REC;
-  // records four at a time, their loads issued together (slots past nblk
-  // read the last record and are skipped by a select)
-  float M = -INFINITY;
-  for (int b = 0; b < nblk; b += 4) {
-    float m4[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) m4[j] = rec0[(int64_t)min(b + j, nblk - 1) * FH_REC + r];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) M = b + j < nblk ? fmaxf(M, m4[j]) : M;
-  }
+// The values of the 4 columns c.. of one row, given its sums: the n_rep heads
+// of the KV head they belong to get the same ones.
+__device__ __forceinline__ void fh_store(const FhParams &p, int row, int c, float M, float L, float4 A) {
   float4 out = zero4();
-  if (M != -INFINITY) {  // a row with no visible key: the chain's P row is all 0
-    float L = 0.f;
-    float4 A = zero4();
-    for (int b = 0; b < nblk; b += 4) {
-      float m4[4], l4[4];
-      float4 a4[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float *rec = rec0 + (int64_t)min(b + j, nblk - 1) * FH_REC;
-        m4[j] = rec[r];
-        l4[j] = rec[FH_ROWS + r];
-        a4[j] = ld4(rec + 2 * FH_ROWS + r * FH_KVD + c);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (b + j >= nblk) break;
-        const float f = __builtin_amdgcn_exp2f(m4[j] - M);  // a block the row cannot see: 0
-        L = fmaf(l4[j], f, L);
-        A.x = fmaf(a4[j].x, f, A.x); A.y = fmaf(a4[j].y, f, A.y);
-        A.z = fmaf(a4[j].z, f, A.z); A.w = fmaf(a4[j].w, f, A.w);
-      }
-    }
+  // a row with no visible key: the chain's P row is all 0
+  if (p.nan_rows ? M != -INFINITY : L > 0.f) {
     const float inv = 1.f / L;
     out = make_float4(A.x * inv, A.y * inv, A.z * inv, A.w * inv);
   }
-  // KV head g's values go to the n_rep heads of group g
   const int g = c / p.head_dim, d = c - g * p.head_dim;
   float *orow = p.o + (int64_t)row * p.ldo + (int64_t)g * p.n_rep * p.head_dim + d;
   for (int h = 0; h < p.n_rep; ++h) *reinterpret_cast<float4 *>(orow + (int64_t)h * p.head_dim) = out;
+}
+
+__global__ __launch_bounds__(64 * FH_WAVES, 2) void fh_rows_kernel(FhParams p) {
+  constexpr int QS = FH_KVD + 4;   // row stride of the group sums: 16 rows on 64 different banks
+  constexpr int OS = FH_KVD / 2 + 4;
+  __shared__ float qsum[FH_ROWS * QS];
+  __shared__ float2 ml[FH_WAVES][FH_ROWS];
+  __shared__ float obuf[FH_WAVES][FH_ROWS * OS];
+  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, r16 = lane & 15, kq = lane >> 4;
+  const int split = blockIdx.x % p.n_split;
+  const int n_rt = (p.sq + FH_ROWS - 1) / FH_ROWS;
+  const int rt = n_rt - 1 - blockIdx.x / p.n_split;  // the rows that see most keys first
+  const int row0 = rt * FH_ROWS;
+  const int kend = fh_key_end(p, min(row0 + FH_ROWS, p.sq) - 1);
+  const int chunk = fh_chunk(p, kend);
+  const int kbeg = split * chunk, kstop = min(kend, kbeg + chunk);
+  if (kbeg >= kend && split > 0) return;  // no record: the merge counts them the same way
+
+  // A operand of S^T: key kt + r16, contraction step (4u + e, kq) = column 16u + 4kq + e
+  float4 kr[16];
+  auto load_k = [&](int kt) __attribute__((always_inline)) {
+    const float *kp = p.k + (int64_t)min(kt + r16, kstop - 1) * p.ldk + 4 * kq;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) kr[u] = ld4(kp + 16 * u);
+  };
+  int kt = kbeg + FH_TILE * w;
+
+  // the group sums of rows 2w, 2w + 1: lane = 4 columns, heads in order
+  {
+    const int c = 4 * lane, g = c / p.head_dim, col = c + g * (p.n_rep - 1) * p.head_dim;
+    float4 a[2];
+    const float *qr[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) qr[i] = p.q + (int64_t)min(row0 + 2 * w + i, p.sq - 1) * p.ldq + col;
+    for (int r0 = 0; r0 < p.n_rep; r0 += kRepChunk) {
+      float4 x[kRepChunk][2];
+#pragma unroll
+      for (int r = 0; r < kRepChunk; ++r)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) x[r][i] = ld4(qr[i] + (int64_t)min(r0 + r, p.n_rep - 1) * p.head_dim);
+      if (r0 == 0 && kt < kstop) load_k(kt);
+#pragma unroll
+      for (int r = 0; r < kRepChunk; ++r) {
+        if (r0 + r >= p.n_rep) break;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          if (r0 + r == 0) {
+            a[i] = x[r][i];
+          } else {
+            a[i].x += x[r][i].x; a[i].y += x[r][i].y; a[i].z += x[r][i].z; a[i].w += x[r][i].w;
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      *reinterpret_cast<float4 *>(&qsum[(2 * w + i) * QS + c]) =
+          make_float4(a[i].x * p.c2, a[i].y * p.c2, a[i].z * p.c2, a[i].w * p.c2);
+  }
+  __syncthreads();
+
+  // O^T: register i of o[t][e] = value column 64t + 16kq + 4i + e of query r16
+  fh_f32x4 o[4][4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[t][e] = fh_f32x4{};
+  const int kend_row = row0 + r16 < p.sq ? min(fh_key_end(p, row0 + r16), kstop) : 0;
+  float m = -INFINITY, l = 0.f;
+  for (; kt < kstop; kt += FH_TILE * FH_WAVES) {
+    asm volatile("" ::: "memory");  // the group sums are read again in each step: kept, they would spill
+    // A operand of P.V: value column 64t + 4 r16 + e (tile (t, e)), key kt + 4kq + i
+    float4 vr[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float *vp = p.v + (int64_t)min(kt + 4 * kq + i, kstop - 1) * p.ldv + 4 * r16;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) vr[i][t] = ld4(vp + 64 * t);
+    }
+    fh_f32x4 s4[4] = {fh_f32x4{}, fh_f32x4{}, fh_f32x4{}, fh_f32x4{}};
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      const float4 b = *reinterpret_cast<const float4 *>(&qsum[r16 * QS + 16 * u + 4 * kq]);
+      fh_f32x4 &s = s4[u & 3];
+      s = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[u].x, b.x, s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[u].y, b.y, s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[u].z, b.z, s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[u].w, b.w, s, 0, 0, 0);
+    }
+    if (kt + FH_TILE * FH_WAVES < kstop) load_k(kt + FH_TILE * FH_WAVES);
+    // register i: key kt + 4kq + i of query r16
+    float pr[4], mx = m;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float x = (s4[0][i] + s4[1][i]) + (s4[2][i] + s4[3][i]);
+      pr[i] = kt + 4 * kq + i < kend_row ? x : -INFINITY;
+      mx = fmaxf(mx, pr[i]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float mu = mx == -INFINITY ? 0.f : mx;
+    const float al = __builtin_amdgcn_exp2f(m - mu);  // no key so far: 0
+    m = mx;
+    l *= al;  // the lane's own 4 keys of each tile
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      pr[i] = __builtin_amdgcn_exp2f(pr[i] - mu);
+      l += pr[i];
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[t][e] *= al;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        o[t][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[i][t].x, pr[i], o[t][0], 0, 0, 0);
+        o[t][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[i][t].y, pr[i], o[t][1], 0, 0, 0);
+        o[t][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[i][t].z, pr[i], o[t][2], 0, 0, 0);
+        o[t][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[i][t].w, pr[i], o[t][3], 0, 0, 0);
+      }
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (kq == 0) ml[w][r16] = make_float2(m, l);
+
+  // the waves' shares meet in LDS, half of the columns at a time; thread =
+  // 4 columns of one row (a wave: two rows)
+  const int row = tid >> 5, c = 4 * (tid & 31);
+  float M = -INFINITY, L = 0.f, f[FH_WAVES];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    if (h) __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<float4 *>(&obuf[w][r16 * OS + 64 * t + 16 * kq + 4 * i]) =
+            make_float4(o[2 * h + t][0][i], o[2 * h + t][1][i], o[2 * h + t][2][i], o[2 * h + t][3][i]);
+    __syncthreads();
+    if (h == 0) {
+      float2 x[FH_WAVES];
+#pragma unroll
+      for (int j = 0; j < FH_WAVES; ++j) x[j] = ml[j][row];
+#pragma unroll
+      for (int j = 0; j < FH_WAVES; ++j) M = fmaxf(M, x[j].x);
+      const float mu = M == -INFINITY ? 0.f : M;
+#pragma unroll
+      for (int j = 0; j < FH_WAVES; ++j) {
+        f[j] = __builtin_amdgcn_exp2f(x[j].x - mu);
+        L = fmaf(x[j].y, f[j], L);
+      }
+    }
+    float4 A = zero4();
+#pragma unroll
+    for (int j = 0; j < FH_WAVES; ++j) {
+      const float4 a = *reinterpret_cast<const float4 *>(&obuf[j][row * OS + c]);
+      A.x = fmaf(a.x, f[j], A.x); A.y = fmaf(a.y, f[j], A.y);
+      A.z = fmaf(a.z, f[j], A.z); A.w = fmaf(a.w, f[j], A.w);
+    }
+    if (row0 + row >= p.sq) continue;
+    if (p.direct) {
+      fh_store(p, row0 + row, 128 * h + c, M, L, A);
+    } else {
+      float *rec = p.rec + (int64_t)(row0 + row) * p.ldr;
+      *reinterpret_cast<float4 *>(rec + FH_KVD * split + 128 * h + c) = A;
+      if (h == 0 && c == 0) *reinterpret_cast<float2 *>(rec + p.ml + 2 * split) = make_float2(M, L);
+    }
+  }
+}
+
+// One wave per row (lane = 4 columns): all of the row's records are in
+// registers before its first store, so they may lie in the row itself.
+__global__ __launch_bounds__(256) void fh_merge_kernel(FhParams p) {
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), c = 4 * (threadIdx.x & 63);
+  if (row >= p.sq) return;
+  const int kend = fh_key_end(p, min(row / FH_ROWS * FH_ROWS + FH_ROWS, p.sq) - 1);
+  const int chunk = fh_chunk(p, kend);
+  const int n = kend > 0 ? (kend + chunk - 1) / chunk : 1;  // the splits that wrote a record
+  const float *rec = p.rec + (int64_t)row * p.ldr;
+  float2 x[FH_SPLITS];
+  float4 a[FH_SPLITS];
+#pragma unroll
+  for (int j = 0; j < FH_SPLITS; ++j) {
+    const int b = min(j, n - 1);
+    x[j] = *reinterpret_cast<const float2 *>(rec + p.ml + 2 * b);
+    a[j] = ld4(rec + FH_KVD * b + c);
+  }
+  float M = -INFINITY, L = 0.f;
+#pragma unroll
+  for (int j = 0; j < FH_SPLITS; ++j) M = fmaxf(M, x[j].x);
+  const float mu = M == -INFINITY ? 0.f : M;
+  float4 A = zero4();
+#pragma unroll
+  for (int j = 0; j < FH_SPLITS; ++j) {
+    if (j >= n) break;
+    const float f = __builtin_amdgcn_exp2f(x[j].x - mu);  // a split the row cannot see: 0
+    L = fmaf(x[j].y, f, L);
+    A.x = fmaf(a[j].x, f, A.x); A.y = fmaf(a[j].y, f, A.y);
+    A.z = fmaf(a[j].z, f, A.z); A.w = fmaf(a[j].w, f, A.w);
+  }
+  fh_store(p, row, c, M, L, A);
+}
+
+// Bytes that a view's elements cover, [lo, hi).
+struct Extent {
+  uintptr_t lo, hi;
+};
+Extent extent(const bn_view *v) {
+  if (v->h == 0 || v->w == 0) return {0, 0};
+  const int64_t first = v->offset, rows = (int64_t)(v->h - 1) * v->stride_h;
+  const int64_t lo = first + std::min<int64_t>(rows, 0), hi = first + std::max<int64_t>(rows, 0) + v->w;
+  const uintptr_t base = reinterpret_cast<uintptr_t>(v->data);
+  return {base + lo * sizeof(float), base + hi * sizeof(float)};
+}
+bool overlaps(const bn_view *a, const bn_view *b) {
+  const Extent x = extent(a), y = extent(b);
+  return x.lo < y.hi && y.lo < x.hi;
+}
+
+// From this many rows a call may take pool memory, and a row whose sum is NaN
+// comes out as NaN; shorter calls take none and give zeros, as the VALU kernel.
+constexpr int kPoolRows = 512;
+// Up to this many keys a call shorter than that stays with the VALU kernel: two
+// key tiles there take less than a second launch (128 rows of 128 keys 12.4 us
+// against 13.0; of 140 keys 15.6 against 12.9).
+constexpr int kValuKeys = 128;
+
+// Splits of a row block's keys.  Up to 36 row blocks, all of them at seven
+// splits are on the card at once; more row blocks fill it with fewer splits,
+// and four (two) are left for their unequal lengths under the causal mask.
+// Measured, us per call, no past, 7 / 6 / 4 / 2 / 1 splits: 384 rows 15.0 /
+// 16.6 / 16.7 / 19.5 / 25.3; 600 rows - / 19.4 / 20.4 / 25.7 / 34.3; 1024
+// rows 29.8 / 28.6 / 27.3 / 35.3 / 49.4; 2048 rows 66 / 60 / 50 / 59 / 89;
+// 4096 rows - / 153 / 132 / 115 / 166; 8192 rows - / 453 / 408 / 375 / 350.
+int fh_splits(int n_rt, int tiles) {
+  const int n = n_rt <= 36 ? 7 : n_rt <= 42 ? 6 : n_rt <= 160 ? 4 : n_rt < 512 ? 2 : 1;
+  return std::max(1, std::min(n, tiles));
+}
+
+int launch_rows(const bn_view *q, const bn_view *k, const bn_view *v, const bn_view *o, int head_dim,
+                int n_rep, float scale, int causal, int seq_offset, hipStream_t s, bool alias) {
+  FhParams f;
+  f.q = reinterpret_cast<const float *>(q->data) + q->offset;
+  f.k = reinterpret_cast<const float *>(k->data) + k->offset;
+  f.v = reinterpret_cast<const float *>(v->data) + v->offset;
+  f.o = reinterpret_cast<float *>(o->data) + o->offset;
+  f.ldq = q->stride_h; f.ldk = k->stride_h; f.ldv = v->stride_h; f.ldo = o->stride_h;
+  f.sq = q->h; f.sk = k->h;
+  f.head_dim = head_dim; f.n_rep = n_rep;
+  f.causal = causal ? 1 : 0;
+  f.seq_offset = seq_offset;
+  f.c2 = scale * 1.4426950408889634f;
+  f.nan_rows = q->h >= kPoolRows;
+  const int n_rt = (q->h + FH_ROWS - 1) / FH_ROWS, tiles = (k->h + FH_TILE - 1) / FH_TILE;
+  const int want = fh_splits(n_rt, tiles);
+  // The records lie in the output's own rows ([split][256], the last 256 for
+  // the (m, l) pairs): an allocation and its release cost 13 us per call.  Pool
+  // memory only where the output overlaps an input, or where the rows' room
+  // leaves fewer splits than wanted and those cost more (a round of the 8 waves
+  // takes 4.6 us: 512 rows + 8000 past, 328 us at one split and 67 at seven).
+  const int room = std::max(1, n_rep - 1);
+  const bool mem = alias || (q->h >= kPoolRows && want > room &&
+                             (int64_t)tiles * (want - room) > 24 * (int64_t)want * room);
+  f.n_split = mem ? want : std::min(want, room);
+  f.direct = f.n_split == 1 && !alias;
+  f.rec = f.o; f.ldr = f.ldo;
+  f.ml = FH_KVD * (mem ? f.n_split : room);
+  void *ws = nullptr;
+  int st;
+  if (mem && !f.direct) {
+    f.ldr = f.ml + 2 * FH_SPLITS + 2;
+    if ((st = bn_alloc(&ws, (size_t)q->h * f.ldr * sizeof(float), s))) return st;
+    f.rec = (float *)ws;
+  }
+  hipLaunchKernelGGL(fh_rows_kernel, dim3((unsigned)((int64_t)n_rt * f.n_split)), dim3(64 * FH_WAVES), 0, s, f);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess && !f.direct) {
+    hipLaunchKernelGGL(fh_merge_kernel, dim3((unsigned)((q->h + 3) / 4)), dim3(256), 0, s, f);
+    e = hipGetLastError();
+  }
+  st = e == hipSuccess ? BN_OK : hip_fail(e, __FILE__, __LINE__);
+  if (!ws) return st;
+  const int st2 = bn_free(ws, s);
+  return st ? st : st2;
 }
 
 // A view the kernel can read with float4 loads: fp32, columns contiguous,
@@ -556,42 +675,10 @@ extern "C" int bn_fused_head_attention(const bn_view *q, const bn_view *k, const
                 std::string(op) + ": views need contiguous columns and rows on 16-byte boundaries");
   if ((st = ensure_device())) return st;
   if (q->h == 0) return BN_OK;
-  if (kvd == FH_KVD && q->h >= kMfmaMinRows) {  // the matrix-core path
-    FhParams f;
-    f.q = reinterpret_cast<const float *>(q->data) + q->offset;
-    f.k = reinterpret_cast<const float *>(k->data) + k->offset;
-    f.v = reinterpret_cast<const float *>(v->data) + v->offset;
-    f.o = reinterpret_cast<float *>(o->data) + o->offset;
-    f.ldq = q->stride_h; f.ldk = k->stride_h; f.ldv = v->stride_h; f.ldo = o->stride_h;
-    f.sq = q->h; f.sk = k->h;
-    f.n_heads = n_heads; f.head_dim = head_dim; f.n_rep = n_heads / n_kv_heads;
-    f.n_kc = (k->h + FH_KEYS - 1) / FH_KEYS;
-    f.causal = causal ? 1 : 0;
-    f.seq_offset = seq_offset;
-    f.c2 = scale * 1.4426950408889634f;
-    const int n_rt = (q->h + FH_ROWS - 1) / FH_ROWS;
-    const size_t qs_bytes = (size_t)q->h * FH_KVD * sizeof(float);
-    const size_t part_bytes = (size_t)n_rt * std::max(f.n_kc, 1) * FH_REC * sizeof(float);
-    void *ws = nullptr;
-    if ((st = bn_alloc(&ws, qs_bytes + part_bytes, stream))) return st;
-    f.qs = (float *)ws;
-    f.part = (float *)((char *)ws + qs_bytes);
-    hipStream_t s = as_stream(stream);
-    const unsigned nvec = (unsigned)(((int64_t)q->h * (FH_KVD / 4) + 255) / 256);
-    hipLaunchKernelGGL(fh_qsum_kernel, dim3(nvec), dim3(256), 0, s, f);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess && f.n_kc > 0) {
-      hipLaunchKernelGGL(fh_mfma_kernel, dim3((unsigned)(n_rt * f.n_kc)), dim3(256), 0, s, f);
-      e = hipGetLastError();
-    }
-    if (e == hipSuccess) {
-      hipLaunchKernelGGL(fh_merge_kernel, dim3(nvec), dim3(256), 0, s, f);
-      e = hipGetLastError();
-    }
-    st = e == hipSuccess ? BN_OK : hip_fail(e, __FILE__, __LINE__);
-    const int st2 = bn_free(ws, stream);
-    return st ? st : st2;
-  }
+  const bool alias = overlaps(o, q) || overlaps(o, k) || overlaps(o, v) || std::abs(o->stride_h) < hd;
+  if (kvd == FH_KVD && (q->h >= kPoolRows || (k->h > kValuKeys && !alias)))
+    return launch_rows(q, k, v, o, head_dim, n_heads / n_kv_heads, scale, causal, seq_offset,
+                       as_stream(stream), alias);
   FusedHeadParams p;
   p.q = reinterpret_cast<const float *>(q->data) + q->offset;
   p.k = reinterpret_cast<const float *>(k->data) + k->offset;

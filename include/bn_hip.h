@@ -179,12 +179,12 @@ int bn_repeat_kv(const bn_view *kv, const bn_view *out, int head_dim, int n_rep,
  * iff j <= i + seq_offset); a row with no visible key is written as zeros, as
  * the chain's all-zero probability row gives.  Needs head_dim % 4 == 0 and
  * n_kv_heads*head_dim a multiple of 16, at most 512.  Results agree with the
- * chain to fp32 rounding (the sums associate differently).  From 512 rows of
- * q with n_kv_heads*head_dim = 256 the call runs on the matrix cores in three
- * launches and takes a stream-ordered pool allocation for the group sums of q
- * and the key blocks' records (seq_q*1 KB plus ~33 KB per 32 x 128 block),
- * released on the same stream; shorter prompts take one launch and no
- * memory. */
+ * chain to fp32 rounding (the sums associate differently).  With
+ * n_kv_heads*head_dim = 256 and more than 128 keys the call runs on the matrix
+ * cores in up to two launches; between them the output's own rows hold partial
+ * sums.  Only a call of 512 rows or more takes a stream-ordered pool
+ * allocation (seq_q * up to 7.3 KB, released on the same stream), and only if
+ * its output overlaps an input or n_rep is below 8 with many keys. */
 int bn_fused_head_attention(const bn_view *q, const bn_view *k, const bn_view *v,
                             const bn_view *o, int n_heads, int n_kv_heads,
                             int head_dim, float scale, int causal, int seq_offset,

@@ -172,3 +172,43 @@ def test_fused_head_attention_matrix_core_views_and_repeats():
     assert np.isnan(got[:, :32]).all() and np.isnan(got[:, 32 + H * D:]).all()
     run(*args, out=out)
     assert np.array_equal(host(big), got, equal_nan=True)
+
+
+@pytest.mark.parametrize("Sq,Sk,H,Hkv,D,causal,off,alias", [
+    (1, 129, 32, 4, 64, True, 128, False),     # one row; the fewest keys of the path, a ragged tile
+    (16, 144, 32, 4, 64, True, 128, False),    # one whole row block, whole tiles
+    (17, 300, 32, 4, 64, True, 290, False),    # one row past it; keys past the last causal one
+    (40, 300, 32, 4, 64, True, -20, False),    # rows 0..19 see no key, their block one or none
+    (200, 200, 8, 8, 32, True, 0, False),      # n_rep 1: the block writes the output itself
+    (130, 200, 16, 8, 32, False, 0, False),    # n_rep 2: room for one record
+    (200, 1000, 12, 4, 64, False, 0, False),   # n_rep 3: two records of the seven
+    (512, 512, 8, 8, 32, True, 0, False),      # n_rep 1, 512 rows: records in pool memory
+    (577, 577, 32, 4, 64, True, 0, False),     # 37 row blocks: six splits
+    (300, 300, 32, 4, 64, True, 0, True),      # the output is the query
+    (520, 520, 32, 4, 64, True, 0, True),      # the same, records in pool memory
+])
+def test_fused_head_attention_key_splits(Sq, Sk, H, Hkv, D, causal, off, alias):
+    """The matrix-core path's row blocks, key splits and homes of their records,
+    the output between guard columns: all n_rep copies equal, the guards
+    untouched, and the rows at both ends against the oracle chain."""
+    r = np.random.default_rng(Sq * 11 + Sk)
+    q = r.standard_normal((Sq, H * D)).astype(np.float32)
+    k = r.standard_normal((Sk, Hkv * D)).astype(np.float32)
+    v = r.standard_normal((Sk, Hkv * D)).astype(np.float32)
+    sc = 1.0 / np.sqrt(D)
+    big = torch.full((Sq, H * D + 8), float("nan"), device="cuda")
+    out = big[:, 4:4 + H * D]
+    if alias:
+        out.copy_(dev(q))
+    run(out if alias else dev(q), dev(k), dev(v), H, Hkv, D, sc, causal, off, out=out)
+    got = host(big)
+    assert np.isnan(got[:, :4]).all() and np.isnan(got[:, 4 + H * D:]).all()
+    got = got[:, 4:4 + H * D]
+    heads = got.reshape(Sq, Hkv, H // Hkv, D)
+    assert (heads == heads[:, :, :1]).all()
+    if off < 0:
+        assert not got[:-off].any()
+    n = min(Sq, 40)
+    for i0 in {0, Sq - n}:
+        ref = O.fused_head_attention(q[i0:i0 + n], k, v, D, H // Hkv, sc, causal, i0 + off)
+        assert_close(got[i0:i0 + n], ref, FP32_TOL, f"rows {i0}..{i0 + n - 1}")
