@@ -733,7 +733,13 @@ __global__ __launch_bounds__(64 * HW * KW, OCC) void prefill_bf16_ks_kernel(Pref
   if (NB > 1 && ni > 0) lstore(0);
   if constexpr (NB > 1) __syncthreads();
   for (int i = 0; i < ni; ++i) {
-    if constexpr (NB == 1) lstore(i);
+    if constexpr (NB == 1) {
+      // the wave's own tile: its LDS instructions execute in order, the
+      // barriers keep the compiler from moving them across
+      __builtin_amdgcn_wave_barrier();
+      lstore(i);
+      __builtin_amdgcn_wave_barrier();
+    }
     gload(i + 1);  // past the range: an empty descriptor, no memory read
     const bf16_t *const kl = smem + (kw * NB + (NB > 1 ? i & 1 : 0)) * (KT + VT), *const vl = kl + KT;
     const int kb = 32 * (kw + KW * i);
@@ -1056,8 +1062,11 @@ __global__ __launch_bounds__(64 * KW, 2) void prefill_f32_ks_kernel(PrefillParam
   f32x16_t o[2] = {f32x16_t{}, f32x16_t{}};  // o[j] row i is d = 2i + j
 
   for (int t = kw; t < nt; t += KW) {
+    // the wave's own tile (barriers as in the bf16 kernel)
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int j = 0; j < 8; ++j) *(u32x4_t *)(kl + (4 * j + (lane >> 4)) * KP + (lane & 15) * 4) = kr[j];
+    __builtin_amdgcn_wave_barrier();
     // this tile's V: key slot (hf, i) of the P V contraction is key 8(i/4) + 4hf + i%4
     float2 vr[16];
     {
