@@ -647,6 +647,9 @@ __global__ __launch_bounds__(64 * NW) void decode_bf16_whole_kernel(DecodeParams
         } while (!__hip_atomic_compare_exchange_strong(word + 1, &old, next, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                        __HIP_MEMORY_SCOPE_AGENT));
         last = (int)(next & 0xffff) == nvalid;
+        // a replay has the same tag: nothing of this count may be left for one
+        // that finds only the first word overwritten
+        if (last) __hip_atomic_store(word + 1, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
       if (last) __hip_atomic_store(word, kArrive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       last_split = last;

@@ -755,3 +755,28 @@ def test_decode_bf16_split_in_one_launch(case):
         for _ in check(50 + n, f"replay {n}"):
             graph.replay()
         run()
+
+
+def test_decode_bf16_split_replay_after_half_a_word_is_overwritten():
+    # every replay has the launch's tag: a count that an earlier replay finished must not be taken for
+    # the start of this one's when another user of the workspace wrote over the first word alone
+    Bn, Lmax, H, Hkv = 3, 2048, 8, 2
+    lens = np.array([2048, 700, 1300], np.int32)
+    q = draw((Bn, H, 64), 61, "bf16")
+    k, v = (draw((Bn, Lmax, Hkv, 64), 62 + i, "bf16") for i in range(2))
+    qd, kd, vd = (dev(x, torch.bfloat16) for x in (q, k, v))
+    ld = torch.tensor(lens, device="cuda")
+    ws = torch.zeros((B.decode_workspace(Bn, Lmax, H).numel() + 7) // 8 * 8, dtype=torch.uint8, device="cuda")
+    first = ws.view(torch.int64)[-2 * Bn * Hkv::2]
+    o = torch.empty_like(qd)
+    run = lambda: B.gqa_decode(qd, kd, vd, ld, o, scale=0.125, workspace=ws)
+    run()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run()
+    ref = O.gqa_decode(q, k, v, lens, 0.125)
+    for n in range(4):
+        first.fill_(n)
+        o.zero_()
+        graph.replay()
+        assert_close(host(o), ref, BF16_TOL, f"replay {n}")
