@@ -467,10 +467,13 @@ __global__ __launch_bounds__(256, OCC) void linear_mn_kernel(LinParams p, RopeFr
 #pragma unroll
     for (int i = 0; i < MF; ++i) {
       const float4 x = make_float4(acc[f][i][0], acc[f][i][1], acc[f][i][2], acc[f][i][3]);
-      const float s0 = r0 ? ta[i].x : 0.f, c0 = r0 ? ta[i].y : 1.f, s1 = r1 ? tb[i].x : 0.f, c1 = r1 ? tb[i].y : 1.f;
+      // columns that do not rotate are selected, not multiplied by (1, 0): an
+      // infinite one would make its neighbour NaN
+      const float y0 = r0 ? x.x * ta[i].y - x.y * ta[i].x : x.x, y1 = r0 ? x.x * ta[i].x + x.y * ta[i].y : x.y;
+      const float y2 = r1 ? x.z * tb[i].y - x.w * tb[i].x : x.z, y3 = r1 ? x.z * tb[i].x + x.w * tb[i].y : x.w;
       typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-      const u32x2_t v = {(uint32_t)f32_to_bf16(x.x * c0 - x.y * s0) | ((uint32_t)f32_to_bf16(x.x * s0 + x.y * c0) << 16),
-                         (uint32_t)f32_to_bf16(x.z * c1 - x.w * s1) | ((uint32_t)f32_to_bf16(x.z * s1 + x.w * c1) << 16)};
+      const u32x2_t v = {(uint32_t)f32_to_bf16(y0) | ((uint32_t)f32_to_bf16(y1) << 16),
+                         (uint32_t)f32_to_bf16(y2) | ((uint32_t)f32_to_bf16(y3) << 16)};
       const int off = ((m_off + 16 * i + l16) * (int)p.y_rs + gn) * 2;
       __builtin_amdgcn_raw_buffer_store_b64(v, ry, gn < p.n ? off : OOB, 0, 0);
     }

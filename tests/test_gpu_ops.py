@@ -562,3 +562,20 @@ def test_linear_rope_bf16_many_rows(case):
     got = host(yb)
     assert_close(got[:, 8:8 + N], O.linear_rope(x, w, rc, off, hd, 1e4), BF16_TOL, f"many rows {case}")
     assert np.all(got[:, :8] == 7.0) and np.all(got[:, 8 + N:] == 7.0)
+
+
+def test_linear_rope_bf16_many_rows_infinite_column():
+    # an infinite column past the rotated ones leaves its neighbours as they are
+    M, K, N, rc = 512, 64, 2560, 1280
+    r = rng(67)
+    x = bf16_round(np.abs(r.standard_normal((M, K))).astype(np.float32) + 0.5)
+    w = bf16_round((r.standard_normal((K, N)) / np.sqrt(K)).astype(np.float32))
+    ref = O.linear_rope(x, w, rc, 0, 64, 1e4)
+    bad = [rc + 1, rc + 6, N - 1]
+    w[:, bad] = np.inf
+    y = torch.empty((M, N), device="cuda", dtype=torch.bfloat16)
+    B.linear_rope(dev(x, torch.bfloat16), dev(w, torch.bfloat16), y, rope_cols=rc, head_dim=64)
+    got = host(y)
+    assert np.all(got[:, bad] == np.inf)
+    rest = np.setdiff1d(np.arange(N), bad)
+    assert_close(got[:, rest], ref[:, rest], BF16_TOL, "beside an infinite column")
