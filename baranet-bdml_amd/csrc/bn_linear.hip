@@ -1138,10 +1138,23 @@ int nt_run(const bn_view *x, const bn_view *w, const bn_view *y, int rope_cols, 
 // x 1536 7.8 / 8.4, 100 x 1536 10.2 / 8.4; K 4096, 250 x 1536 20.3 / 23.7,
 // 200 x 3072 25.0 / 26.4, 250 x 3072 26.9 / 26.6, 700 x 1536 35.3 / 30.6;
 // K 5632, 320 x 2048 27.9 / 31.7).
-bool mn_takes(int m, int n, int k, int64_t x_rs, int64_t w_rs, int64_t y_rs) {
+// Rows that overlap, repeat or run backwards (strides below the width) stay
+// with the other kernels, whose addresses are not bounded by a descriptor over
+// whole rows; so does a y that overlaps x or w, which split-k writes only
+// after its last read.
+bool mn_takes(const bn_view *x, const bn_view *w, const bn_view *y) {
   constexpr int64_t kMaxRs = 1 << 21;  // 160 rows of a tile stay below 2^30 bytes
+  const int m = y->h, n = w->w, k = x->w;
   const int64_t least = 48 + (k > 2048 ? (k - 2048) / 8 : 0);
-  return k > 0 && m >= 48 && (int64_t)m * n >= 2560 * least && x_rs < kMaxRs && w_rs < kMaxRs && y_rs < kMaxRs;
+  if (k <= 0 || m < 48 || (int64_t)m * n < 2560 * least) return false;
+  for (const bn_view *v : {x, w, y})
+    if ((v->h > 1 && v->stride_h < v->w) || v->stride_h < 0 || v->stride_h >= kMaxRs) return false;
+  auto apart = [](const bn_view *a, const bn_view *b) {
+    auto lo = [](const bn_view *v) { return (uintptr_t)v->data + v->offset * sizeof(bf16_t); };
+    auto hi = [&](const bn_view *v) { return lo(v) + ((int64_t)(v->h - 1) * v->stride_h + v->w) * sizeof(bf16_t); };
+    return hi(a) <= lo(b) || hi(b) <= lo(a);
+  };
+  return apart(y, x) && apart(y, w);
 }
 int mn_run(const bn_view *x, const bn_view *w, const bn_view *y, int rope_cols, int position_offset,
            int head_dim, const RopeFreqs &fr, hipStream_t s) {
@@ -1361,7 +1374,7 @@ int linear_run(const bn_view *x, const bn_view *w, const bn_view *y, int rope_co
     return fail(BN_ERR_UNSUPPORTED, std::string(op) + ": problem too large");
   if ((st = ensure_device())) return st;
   hipStream_t s = as_stream(stream);
-  if (dt == BN_BF16 && epi == EPI_PLAIN && !k_dst && mn_takes(m, n, k, x->stride_h, w->stride_h, y->stride_h))
+  if (dt == BN_BF16 && epi == EPI_PLAIN && !k_dst && mn_takes(x, w, y))
     return mn_run(x, w, y, rope_cols, position_offset, head_dim, fr, s);
   void *ws = workspace;
   bool own = false;

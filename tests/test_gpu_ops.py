@@ -579,3 +579,18 @@ def test_linear_rope_bf16_many_rows_infinite_column():
     assert np.all(got[:, bad] == np.inf)
     rest = np.setdiff1d(np.arange(N), bad)
     assert_close(got[:, rest], ref[:, rest], BF16_TOL, "beside an infinite column")
+
+
+@pytest.mark.parametrize("form", ["windows", "one_row", "in_place"])
+def test_linear_bf16_many_rows_other_layouts(form):
+    # rows that overlap or repeat, and a y that lies over x: not the descriptor kernel's
+    M, K, N = 256, 512, 512
+    r = rng(68)
+    w = bf16_round((r.standard_normal((K, N)) / np.sqrt(K)).astype(np.float32))
+    rs = {"windows": 16, "one_row": 0, "in_place": K}[form]
+    buf = dev(bf16_round(r.standard_normal((M - 1) * rs + K).astype(np.float32)), torch.bfloat16)
+    xd = buf.as_strided((M, K), (rs, 1))
+    ref = O.linear_rope(host(xd.contiguous()), w, 0, 0, 64, 1e4)
+    y = xd if form == "in_place" else torch.empty((M, N), device="cuda", dtype=torch.bfloat16)
+    B.linear_rope(xd, dev(w, torch.bfloat16), y, rope_cols=0, head_dim=64)
+    assert_close(host(y), ref, BF16_TOL, form)
