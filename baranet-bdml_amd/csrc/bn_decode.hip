@@ -540,8 +540,8 @@ __global__ __launch_bounds__(64 * NW) void decode_bf16_whole_kernel(DecodeParams
                      fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float m_new = fmaxf(m, mx);  // finite: every tile holds at least one key
-    const float mc = m_new * c;
+    const float m_new = fmaxf(m, mx);  // -inf while every key so far scores -inf
+    const float mc = (m_new == -INFINITY ? 0.f : m_new) * c;
     const float alpha = __builtin_amdgcn_exp2f(m * c - mc);  // m = -inf -> 0
     float rs = 0.f;
     dbf16x8_t pb;
@@ -611,16 +611,17 @@ __global__ __launch_bounds__(64 * NW) void decode_bf16_whole_kernel(DecodeParams
     const int h = idx / HD, d = idx - h * HD;
     float M = red_m[0][h];
 #pragma unroll
-    for (int w = 1; w < NW; ++w) M = fmaxf(M, red_m[w][h]);  // finite: wave 0 has keys
+    for (int w = 1; w < NW; ++w) M = fmaxf(M, red_m[w][h]);
+    const float Mu = M == -INFINITY ? 0.f : M;  // no key above -inf: every weight 0
     float L = 0.f, A = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-      const float wt = __builtin_amdgcn_exp2f(red_m[w][h] - M);
+      const float wt = __builtin_amdgcn_exp2f(red_m[w][h] - Mu);
       L += red_l[w][h] * wt;
       A += red_o[w][h][d] * wt;
     }
     if (!SPLIT || nvalid == 1) {
-      out[idx] = f32_to_bf16(A / L);
+      out[idx] = f32_to_bf16(L == 0.f ? 0.f : A / L);
     } else {
       float *rec = p.ws + (((int64_t)b * p.n_heads + (int64_t)g * G + h) * p.n_split + split) * kDecRec;
       auto wr = [](float *q, float v) { __hip_atomic_store(q, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); };

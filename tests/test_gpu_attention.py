@@ -780,3 +780,52 @@ def test_decode_bf16_split_replay_after_half_a_word_is_overwritten():
         o.zero_()
         graph.replay()
         assert_close(host(o), ref, BF16_TOL, f"replay {n}")
+
+
+# keys that score -inf for every head (an additive mask carried in the cache: -inf, or the lowest bf16
+# value, whose product with the query overflows) weigh 0, wherever they lie: single keys, a whole
+# 32-key tile, a whole split, the cache's end; a cache of nothing else gives zeros
+MASKED_DECODE_CASES = [
+    # batch, max_len, H, Hkv, head-major
+    (6, 2048, 16, 2, True),     # 12 pairs: eight splits of 256 keys
+    (40, 300, 32, 4, False),    # 160 pairs: unsplit, eight waves
+    (64, 300, 32, 4, True),     # 256 pairs: four waves, six for a long cache
+    (64, 300, 32, 4, False),
+]
+
+
+@pytest.mark.parametrize("mask", [-math.inf, float(torch.finfo(torch.bfloat16).min)])
+@pytest.mark.parametrize("case", MASKED_DECODE_CASES)
+def test_decode_bf16_keys_of_minus_infinity(case, mask):
+    Bn, Lmax, H, Hkv, head_major = case
+    G = H // Hkv
+    q = draw((Bn, H, 64), 71, "bf16")
+    q[:, :, 0] = 2.0 + np.abs(q[:, :, 0])  # the mask's column: score mask * q0 for every head
+    k, v = (draw((Bn, Lmax, Hkv, 64), 72 + i, "bf16") for i in range(2))
+    k[..., 0] = 0.0
+    lens = np.random.default_rng(74).integers(Lmax // 2, Lmax + 1, Bn).astype(np.int32)
+    lens[:6] = [Lmax, Lmax, Lmax - 7, Lmax, 64, Lmax]
+    hidden = np.zeros((Bn, Lmax), bool)
+    hidden[0, 32:64] = True                        # a tile of the first split
+    hidden[1, : Lmax // 8] = True                  # the first split
+    hidden[2, Lmax - 64:] = True                   # the last tiles, one of them ragged
+    hidden[3, :] = True                            # everything
+    hidden[4, :40] = True                          # a tile and a part of the only other one
+    hidden[5, Lmax // 4: Lmax // 2] = True         # two whole splits in the middle
+    hidden[6:, ::3] = True                         # single keys
+    k[hidden, :, 0] = mask
+    cache = [dev(x, torch.bfloat16) for x in (k, v)]
+    if head_major:
+        cache = [x.transpose(1, 2).contiguous().transpose(1, 2) for x in cache]
+    ld = torch.tensor(lens, device="cuda")
+    o = host(B.gqa_decode(dev(q, torch.bfloat16), *cache, ld, scale=0.125))
+    ref = np.zeros((Bn, H, 64))
+    for b in range(Bn):
+        seen = ~hidden[b, : lens[b]]
+        for g in range(Hkv if seen.any() else 0):
+            kk, vv = (x[b, : lens[b], g][seen].astype(np.float64) for x in (k, v))
+            s = q[b, g * G:(g + 1) * G].astype(np.float64) @ kk.T * 0.125
+            e = np.exp(s - s.max(1, keepdims=True))
+            ref[b, g * G:(g + 1) * G] = e / e.sum(1, keepdims=True) @ vv
+    assert_close(o, ref, BF16_TOL, f"masked keys {case} {mask}")
+    assert np.all(o[3] == 0.0)
