@@ -862,8 +862,8 @@ __global__ __launch_bounds__(kPlanThreads) void decode_bf16_planned_kernel(PlanP
                      fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float m_new = fmaxf(m, mx);  // finite: every tile holds at least one key
-    const float mc = m_new * c;
+    const float m_new = fmaxf(m, mx);  // -inf while every key so far scores -inf
+    const float mr = m_new * c, mc = mr == -INFINITY ? 0.f : mr;
     const float alpha = __builtin_amdgcn_exp2f(m * c - mc);  // m = -inf -> 0
     float rs = 0.f;
     dbf16x8_t pb;
@@ -995,7 +995,9 @@ __global__ __launch_bounds__(kPlanThreads) void decode_bf16_planned_kernel(PlanP
     if (polls < kPlanPolls) {
       for (int idx = lane; idx < G * HD; idx += 64) {
         const int h = idx / HD, d = idx - h * HD;
-        float M = red_m[0][0][h];
+        // (a part whose keys all score -inf: a finite M whose sums are 0, so
+        // that the merges subtract finite numbers)
+        float M = fmaxf(red_m[0][0][h], -__FLT_MAX__);
 #pragma unroll
         for (int w = 1; w < WWV; ++w) M = fmaxf(M, red_m[0][w][h]);
         float L = 0.f, A = 0.f;
@@ -1032,12 +1034,11 @@ __global__ __launch_bounds__(kPlanThreads) void decode_bf16_planned_kernel(PlanP
     // this share's waves: (M, L, A) of output idx from LDS slot ls
     auto own = [&](int ls, int idx, float &M, float &L, float &A) __attribute__((always_inline)) {
       const int h = idx / HD, d = idx - h * HD;
-      M = red_m[ls][0][h];
+      M = fmaxf(red_m[ls][0][h], -__FLT_MAX__);  // finite, as the records'
 #pragma unroll
       for (int w = 1; w < WWV; ++w) M = fmaxf(M, red_m[ls][w][h]);
       L = 0.f;
       A = 0.f;
-      if (M == -INFINITY) return;  // no key in any wave (a fallback slot can be empty)
 #pragma unroll
       for (int w = 0; w < WWV; ++w) {
         const float wt = __builtin_amdgcn_exp2f(red_m[ls][w][h] - M);
@@ -1049,7 +1050,7 @@ __global__ __launch_bounds__(kPlanThreads) void decode_bf16_planned_kernel(PlanP
       for (int idx = tid; idx < G * HD; idx += kPlanThreads) {
         float M, L, A;
         own(s, idx, M, L, A);
-        out[idx] = f32_to_bf16(A / L);
+        out[idx] = f32_to_bf16(L == 0.f ? 0.f : A / L);
       }
       continue;
     }
@@ -1083,7 +1084,7 @@ __global__ __launch_bounds__(kPlanThreads) void decode_bf16_planned_kernel(PlanP
         for (int j = 0; j < NO; ++j) {
           ok = ok && (wm[j] >> 32) == p.epoch && (wl[j] >> 32) == p.epoch && (wa[j] >> 32) == p.epoch;
           const float mq = __builtin_bit_cast(float, (uint32_t)wm[j]);
-          const float m2 = fmaxf(Mv[j], mq);  // finite: this share's part has keys
+          const float m2 = fmaxf(Mv[j], mq);
           const float a1 = __builtin_amdgcn_exp2f(Mv[j] - m2), a2 = __builtin_amdgcn_exp2f(mq - m2);
           Lv[j] = Lv[j] * a1 + __builtin_bit_cast(float, (uint32_t)wl[j]) * a2;
           Av[j] = Av[j] * a1 + __builtin_bit_cast(float, (uint32_t)wa[j]) * a2;
@@ -1148,7 +1149,7 @@ __global__ __launch_bounds__(kPlanThreads) void decode_bf16_planned_kernel(PlanP
 #pragma unroll
     for (int j = 0; j < NO; ++j) {
       const int idx = tid + kPlanThreads * j;
-      if (idx < G * HD) out[idx] = f32_to_bf16(Av[j] / Lv[j]);
+      if (idx < G * HD) out[idx] = f32_to_bf16(Lv[j] == 0.f ? 0.f : Av[j] / Lv[j]);
     }
     __syncthreads();  // the fallback's LDS slot and state are reused by the next segment
   }

@@ -144,3 +144,41 @@ def test_planned_decode_fallback_path(kind):
         run_case(Bn, L, H, Hkv, lengths(kind, Bn, L), seed=17)
     finally:
         del os.environ["BN_PLAN_FALLBACK"]
+
+
+@pytest.mark.parametrize("fallback", [False, True])
+def test_planned_decode_keys_of_minus_infinity(fallback):
+    """Keys that score -inf for every head weigh 0: tiles of an uncut cache, the
+    head part, a later part and the whole of cut caches (zeros)."""
+    Bn, L, H, Hkv = 64, 2048, 32, 4
+    G = H // Hkv
+    lens = lengths("skewed", Bn, L)  # caches 3, 20, 41 and 62 of 2048 keys are cut
+    r = np.random.default_rng(23)
+    q, k, v = (bf16_round(r.standard_normal(s).astype(np.float32))
+               for s in ((Bn, H, 64), (Bn, L, Hkv, 64), (Bn, L, Hkv, 64)))
+    q[:, :, 0] = 1.0 + np.abs(q[:, :, 0])
+    k[..., 0] = 0.0
+    hidden = np.zeros((Bn, L), bool)
+    hidden[0, :64] = hidden[1, 256:320] = True
+    hidden[3, :1024] = True
+    hidden[20, 1024:] = True
+    hidden[41, :] = True
+    hidden[7, :] = True
+    k[hidden, :, 0] = -np.inf
+    ld = torch.from_numpy(lens).cuda()
+    if fallback:
+        os.environ["BN_PLAN_FALLBACK"] = "1"
+    try:
+        o = host(B.gqa_decode_planned(*(dev(x, torch.bfloat16) for x in (q, k, v)), ld, lens, scale=0.125))
+    finally:
+        os.environ.pop("BN_PLAN_FALLBACK", None)
+    ref = np.zeros((Bn, H, 64))
+    for b in range(Bn):
+        seen = ~hidden[b, : lens[b]]
+        for g in range(Hkv if seen.any() else 0):
+            kk, vv = (x[b, : lens[b], g][seen].astype(np.float64) for x in (k, v))
+            s = q[b, g * G:(g + 1) * G].astype(np.float64) @ kk.T * 0.125
+            e = np.exp(s - s.max(1, keepdims=True))
+            ref[b, g * G:(g + 1) * G] = e / e.sum(1, keepdims=True) @ vv
+    assert_close(o, ref, BF16_TOL, "masked keys")
+    assert np.all(o[[7, 41]] == 0.0)
