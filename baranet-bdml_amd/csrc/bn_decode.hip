@@ -417,8 +417,12 @@ __device__ __forceinline__ int split_chunk(int len, int n_split) {
 // The arrival words stand at the workspace's end.  The first holds kArrive
 // between calls and counts up from it: one atomic.  Anything else there (a
 // fresh workspace) sends every split of the launch to the second word, where a
-// count starts under the launch's tag: a load and a compare-exchange that the
-// splits contend for (12 caches in 8 splits: 17.4 against 12.2 us).  The last
+// count starts under the launch's tag: a load, for the first splits a
+// compare-exchange, and an add (words overwritten before every call, whose
+// fill is in the time: one cache of 1530 keys 10.2 us, 14066 keys 18.6, four of
+// 4203..7439 16.4; with a compare-exchange per arrival, which all retry while
+// others arrive, 11.6, 20.1 and 18.2; the former chunk kernel 11.5, 22.7 and
+// 18.0).  A finished count clears the second word, and the last
 // arrival leaves kArrive, so neither a fresh workspace nor a replayed graph
 // needs a clearing pass.
 template <int G, int NW, bool SPLIT>
@@ -641,12 +645,14 @@ __global__ __launch_bounds__(64 * NW) void decode_bf16_whole_kernel(DecodeParams
       unsigned long long old = __hip_atomic_fetch_add(word, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       bool last = old - kArrive == (unsigned long long)(nvalid - 1);
       if (old - kArrive >= (unsigned long long)nvalid) {
-        unsigned long long next;
+        // one split puts the tag there, then every split adds
         old = __hip_atomic_load(word + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        do {
-          next = (old >> 16 == p.tag ? old : p.tag << 16) + 1;
-        } while (!__hip_atomic_compare_exchange_strong(word + 1, &old, next, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                       __HIP_MEMORY_SCOPE_AGENT));
+        while (old >> 16 != p.tag &&
+               !__hip_atomic_compare_exchange_strong(word + 1, &old, p.tag << 16, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT)) {
+        }
+        const unsigned long long next =
+            __hip_atomic_fetch_add(word + 1, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
         last = (int)(next & 0xffff) == nvalid;
         // a replay has the same tag: nothing of this count may be left for one
         // that finds only the first word overwritten

@@ -339,9 +339,11 @@ int bn_llama_decode(const bn_llama_config *config, const float *embed,
  * call needs it); single-pass calls use none: bf16 caches with
  * batch*n_kv_heads above half the device's compute units or of at most 256
  * keys.  Other bf16 calls keep split records there and, at its end, arrival
- * words that the splits count in on; a call whose workspace the previous call
- * also used (any shape) finds them ready, and on any other contents the count
- * takes a slower path to the same result.  fp32 caches of at most
+ * words that the splits count in on, two per (sequence, KV head).  A pair
+ * finds its words ready if an earlier call with this workspace (same address
+ * and size) split that pair and nothing has written over them since; on any
+ * other contents its count takes a slightly slower path to the same result.
+ * fp32 caches of at most
  * 1024 keys with batch*n_heads <= 256 keep 4 split records per (sequence,
  * head) in it and merge them in the same launch, counting on a ring of 16
  * counter slots inside the library: at most 16 such calls in flight at once
