@@ -82,12 +82,28 @@ __device__ __forceinline__ float row_sum(float x) {
   return x;
 }
 
+// Sum over the wave, a uniform value, without an LDS round trip: DPP moves inside
+// each 16-lane row, then the rows' sums by readlane.
+template <int CTRL>
+__device__ __forceinline__ int dpp_add(int v) {
+  return v + __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, false);
+}
+__device__ __forceinline__ int wave_sum_i32(int v) {
+  v = dpp_add<0x140>(dpp_add<0x141>(dpp_add<0x4E>(dpp_add<0xB1>(v))));
+  return __builtin_amdgcn_readlane(v, 0) + __builtin_amdgcn_readlane(v, 16) + __builtin_amdgcn_readlane(v, 32) +
+         __builtin_amdgcn_readlane(v, 48);
+}
+
 struct DecodeParams {
   const void *q, *k, *v;
   const int32_t *lens;
   void *o;
   float *ws;  // partials: [batch*n_heads][n_split][HD + 2]
   int batch, max_len, n_heads, n_kv_heads, n_split, chunk;
+  // dealt caches: pieces of a cache at least (n_split: at most), the workgroups
+  // per KV head for further pieces, and whether only far longer caches than the
+  // others get them
+  int min_split = 1, more = 0, outliers = 0;
   float c;        // scale * log2(e)
   int hlen = -1;  // >= 0: every sequence's length, from the host (lens not read)
   // cache strides in elements: sequence, KV head, key row (a contiguous
@@ -393,6 +409,12 @@ constexpr int WKP = HD + 8;  // tile row pitch, 144 B: b128 K reads of 16 rows a
 
 // a cache up to this length is one split's (500 keys: 5.8 us, in 2-8 splits 6.9)
 constexpr int kSplitMinLen = 512;
+// how a cache is dealt to workgroups: whole, in n_split equal pieces, or in
+// pieces that follow its length and the batch's
+constexpr int kWhole = 0, kSplit = 1, kDealt = 2;
+constexpr int kPieceMinLen = 1024;  // keys of a dealt piece at least
+constexpr int kFewPairs = 32;       // below, a cache's pieces follow its own length alone
+constexpr int kDealtMax = 256;      // sequences of a dealt batch (4 a lane)
 constexpr unsigned long long kArrive = 0x5bd1e995a93c71d4ull;
 // keys per split of a cache: whole rounds of the workgroup's four tiles
 template <int NW>
@@ -403,7 +425,8 @@ __device__ __forceinline__ int split_chunk(int len, int n_split) {
 }
 
 // NW waves per workgroup: WWV, or WWX with the long-cache adaptation.
-// SPLIT (fewer (sequence, KV head) pairs than compute units): n_split
+// SPLIT (fewer (sequence, KV head) pairs than compute units; kSplit equal
+// pieces, kDealt by the lengths, dealt_splits): up to n_split
 // workgroups per pair, each over a run of the cache, so that a few caches
 // have most of their loads in flight at once; bound by latencies (launch, one
 // or two memory round trips, the merge).  A split writes its merged (m, l,
@@ -425,8 +448,9 @@ __device__ __forceinline__ int split_chunk(int len, int n_split) {
 // 18.0).  A finished count clears the second word, and the last
 // arrival leaves kArrive, so neither a fresh workspace nor a replayed graph
 // needs a clearing pass.
-template <int G, int NW, bool SPLIT>
+template <int G, int NW, int DEAL>
 __global__ __launch_bounds__(64 * NW) void decode_bf16_whole_kernel(DecodeParams p) {
+  constexpr bool SPLIT = DEAL != kWhole;
   __shared__ __attribute__((aligned(16))) bf16_t KT[NW][TK * WKP];
   __shared__ __attribute__((aligned(16))) bf16_t VT[NW][TK * WKP];
   __shared__ float red_m[NW][G], red_l[NW][G];
@@ -438,7 +462,7 @@ __global__ __launch_bounds__(64 * NW) void decode_bf16_whole_kernel(DecodeParams
   const int l16 = lane & 15, grp = lane >> 4;
   // the KV heads of a sequence's (split's) rows next to each other
   const int g = blockIdx.x % p.n_kv_heads, bs = blockIdx.x / p.n_kv_heads;
-  const int b = SPLIT ? bs / p.n_split : bs, split = SPLIT ? bs - b * p.n_split : 0;
+  int b = SPLIT ? bs / p.n_split : bs, split = SPLIT ? bs - b * p.n_split : 0;
   auto clamp_len = [&](int x) { return x < 0 ? 0 : (x > p.max_len ? p.max_len : x); };
 
   // the batch's total length (batches up to kMeanBatchMax sequences), summed
@@ -447,9 +471,67 @@ __global__ __launch_bounds__(64 * NW) void decode_bf16_whole_kernel(DecodeParams
   int part = 0;
   if (adapt)
     for (int i = lane; i < p.batch; i += 64) part += clamp_len(p.lens[i]);
+  int pieces = SPLIT ? p.n_split : 1;
+  if (DEAL == kDealt && p.batch * p.n_kv_heads >= kFewPairs) {
+    // min_split pieces of every cache first; the p.more workgroups per
+    // KV head after those take the further pieces of the longer caches, found by
+    // a scan over the batch that every wave makes for itself (lane: 4 sequences)
+    int t[4], sum = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int s = 4 * lane + i;
+      t[i] = s < p.batch ? min((clamp_len(p.lens[s]) + TK - 1) / TK, 1 << 22) : 0;
+      sum += t[i];
+    }
+    const int total = wave_sum_i32(sum);  // <= 2^30
+    // A cache has as many pieces as it holds whole shares.  A share is more
+    // than the batch's tiles over p.more, so the caches hold fewer of them than
+    // there are workgroups.
+    const int share = max((int)((uint32_t)total / (uint32_t)p.more) + 1, kPieceMinLen / TK);
+    auto pieces_of = [&](int tiles) {
+      if (p.outliers && (int64_t)tiles * p.batch <= 4 * (int64_t)total) return p.min_split;
+      return min(max((int)((uint32_t)tiles / (uint32_t)share), p.min_split), p.n_split);
+    };
+    const int j = bs - p.batch * p.min_split;
+    if (j < 0) {
+      b = bs / p.min_split;
+      split = bs - b * p.min_split;
+    } else {
+      int more[4], in = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        more[i] = pieces_of(t[i]) - p.min_split;
+        in += more[i];
+      }
+      const int own = in;
+#pragma unroll
+      for (int o2 = 1; o2 < 64; o2 <<= 1) {
+        const int x = __shfl_up(in, o2, 64);
+        in += lane >= o2 ? x : 0;
+      }
+      const uint64_t past = __builtin_amdgcn_ballot_w64(in > j);
+      if (past == 0) return;
+      const int src = __builtin_ctzll(past);
+      int k = j - __shfl(in - own, src, 64);
+      int i = 0;
+#pragma unroll
+      for (int e = 0; e < 3; ++e) {
+        const int n = __shfl(more[e], src, 64);
+        if (i == e && k >= n) {
+          k -= n;
+          ++i;
+        }
+      }
+      b = __builtin_amdgcn_readfirstlane(4 * src + i);
+      split = __builtin_amdgcn_readfirstlane(p.min_split + k);
+    }
+    pieces = pieces_of(min((clamp_len(p.lens[b]) + TK - 1) / TK, 1 << 22));
+  }
   const int len = clamp_len(p.lens[b]);
+  if (DEAL == kDealt && p.batch * p.n_kv_heads < kFewPairs)
+    pieces = min(max(len / kPieceMinLen & ~7, p.min_split), p.n_split);  // (records merge eight at a time)
   bf16_t *out = (bf16_t *)p.o + ((int64_t)b * p.n_heads + (int64_t)g * G) * HD;
-  const int chunk = SPLIT ? split_chunk<NW>(len, p.n_split) : 0;
+  const int chunk = SPLIT ? split_chunk<NW>(len, pieces) : 0;
   const int k0 = split * chunk;
   if (SPLIT && split > 0 && k0 >= len) return;
   if (len == 0) {  // no key: zeros
@@ -1311,6 +1393,36 @@ uint32_t next_plan_epoch() {
 int whole_splits(int units, int max_len) {
   return std::max(1, std::min({256 / units, 8, (max_len + 127) / 128 - 1}));
 }
+// Where caches can be longer than those lines were drawn for, their pieces
+// follow the lengths (kDealt).  Returns the most pieces of a cache, and in more
+// the workgroups per KV head for pieces past whole_splits(), in outliers whether only a
+// cache of more than four times the batch's mean length has any; 0: equal
+// pieces as above.  us, former chunk kernel / equal pieces / dealt, 4 KV heads:
+//  - below 32 pairs (a piece per 1024 keys, in eights since eight records merge
+//    at a time): one cache of 16384 keys 23.4 / 16.8 / 13.4, of 131072 86 / 94 /
+//    32, with 8 KV heads 74 / 97 / 44; of 1543 in 131072 rows 11.8 / 6.9 / 6.9
+//  - to 128 pairs, from 16384 rows: one cache of 32768 among 31 of 500 65 / 95 /
+//    21, 12 token-major caches of 913..32149 56 / 49 / 50 (every cache dealt:
+//    53); where the equal pieces leave a fifth of 256 workgroups unused every
+//    cache is dealt: 24 of 2308..30794 96 / 102 / 70 (32 of 816..30488, which
+//    leave none: 119 / 113 / 162).  32 of 562..16351 57 / 60 / 61 is left.
+//  - to 255 pairs, from 5120 rows: 33 token-major caches of 639..8162 47 / 53 /
+//    32, all of 8192 61 / 58 / 58, 40 of 888..16067 85 / 102 / 71, 56 of
+//    549..5949 39 / 43 / 42; one of 16384 among 39 of 500 42 / 94 / 15.  Eight
+//    waves hold a CU each even where they find no piece, so head-major calls
+//    have 64 workgroups for them (256 cost 63 uniform caches 2.5%): one of 16384
+//    among 39 of 500 45 / 73 / 20.
+// The scan costs 0.6 us: 8 caches of 16384 23.3 / 23.9, 63 of 1000 in 16384 rows
+// 12.6 / 14.2 (99 before).
+int dealt_splits(int batch, int n_kv_heads, int max_len, bool token_major, int *more, int *outliers) {
+  const int units = batch * n_kv_heads, by_len = max_len / kPieceMinLen;
+  *more = *outliers = 0;
+  if (batch > kDealtMax || units >= 256 || by_len < (units > 128 ? 5 : 16)) return 0;
+  if (units < kFewPairs) return std::min({256 / units, 64, by_len & ~7});
+  *more = (units > 128 && !token_major ? 64 : 256) / n_kv_heads;
+  *outliers = units <= 128 && units * whole_splits(units, max_len) > 204;
+  return *more ? std::min(by_len, units > 128 ? 32 : 64) : 0;
+}
 // a launch's 48-bit tag: a mixed counter (SplitMix64's finaliser), so that
 // no plausible memory contents look like this launch's arrivals
 std::atomic<uint64_t> g_split_launch{0};
@@ -1422,9 +1534,9 @@ int gqa_decode_impl(int dtype, const void *q, const void *k_cache, const void *v
 #define BN_WHOLE(GG)                                                                        \
   do {                                                                                      \
     if (wide)                                                                               \
-      hipLaunchKernelGGL((decode_bf16_whole_kernel<GG, WWX, false>), grid, block, 0, s, p);        \
+      hipLaunchKernelGGL((decode_bf16_whole_kernel<GG, WWX, kWhole>), grid, block, 0, s, p);        \
     else                                                                                    \
-      hipLaunchKernelGGL((decode_bf16_whole_kernel<GG, WWV, false>), grid, block, 0, s, p);        \
+      hipLaunchKernelGGL((decode_bf16_whole_kernel<GG, WWV, kWhole>), grid, block, 0, s, p);        \
   } while (0)
       switch (G) {
         case 1: BN_WHOLE(1); break;
@@ -1455,8 +1567,13 @@ int gqa_decode_impl(int dtype, const void *q, const void *k_cache, const void *v
                                         std::to_string((size_t)BN_GQA_DECODE_SCRATCH_BYTES) +
                                         "-byte scratch");
   size_t words = 0;
+  bool dealt = false;
   if (bsplit) {  // (the no-allocation limit above stays that of the chunks' partials)
-    p.n_split = whole_splits(batch * n_kv_heads, max_len);
+    p.min_split = p.n_split = whole_splits(batch * n_kv_heads, max_len);
+    const int most =
+        dealt_splits(batch, n_kv_heads, max_len, p.kv_rs != HD, &p.more, &p.outliers);
+    dealt = most > p.n_split;
+    if (dealt) p.n_split = most;
     words = p.n_split > 1 ? (size_t)batch * n_kv_heads * 16 + 8 : 0;
     need = p.n_split > 1 ? (size_t)batch * n_heads * p.n_split * kDecRec * sizeof(float) + words : 0;
   }
@@ -1482,13 +1599,19 @@ int gqa_decode_impl(int dtype, const void *q, const void *k_cache, const void *v
       p.arrive_end = (unsigned long long *)(((uintptr_t)ws + bytes) & ~(uintptr_t)7);
       p.tag = next_split_tag();
     }
-    const dim3 grid((unsigned)((int64_t)batch * n_kv_heads * p.n_split));
-#define BN_SPLIT(GG)                                                                                  \
-  do {                                                                                                \
-    if (p.n_split > 1)                                                                                \
-      hipLaunchKernelGGL((decode_bf16_whole_kernel<GG, WWV, true>), grid, dim3(64 * WWV), 0, s, p);   \
-    else                                                                                              \
-      hipLaunchKernelGGL((decode_bf16_whole_kernel<GG, WW1, true>), grid, dim3(64 * WW1), 0, s, p);   \
+    const int units = batch * n_kv_heads;
+    const dim3 grid((unsigned)(dealt && p.more ? units * p.min_split + n_kv_heads * p.more : units * p.n_split));
+    const bool eight = dealt ? units > 128 && p.kv_rs == HD : p.n_split == 1;  // waves
+#define BN_SPLIT(GG)                                                                                        \
+  do {                                                                                                      \
+    if (dealt && eight)                                                                                     \
+      hipLaunchKernelGGL((decode_bf16_whole_kernel<GG, WW1, kDealt>), grid, dim3(64 * WW1), 0, s, p);       \
+    else if (dealt)                                                                                         \
+      hipLaunchKernelGGL((decode_bf16_whole_kernel<GG, WWV, kDealt>), grid, dim3(64 * WWV), 0, s, p);       \
+    else if (eight)                                                                                         \
+      hipLaunchKernelGGL((decode_bf16_whole_kernel<GG, WW1, kSplit>), grid, dim3(64 * WW1), 0, s, p);       \
+    else                                                                                                    \
+      hipLaunchKernelGGL((decode_bf16_whole_kernel<GG, WWV, kSplit>), grid, dim3(64 * WWV), 0, s, p);       \
   } while (0)
     switch (G) {
       case 1: BN_SPLIT(1); break;

@@ -829,3 +829,64 @@ def test_decode_bf16_keys_of_minus_infinity(case, mask):
             ref[b, g * G:(g + 1) * G] = e / e.sum(1, keepdims=True) @ vv
     assert_close(o, ref, BF16_TOL, f"masked keys {case} {mask}")
     assert np.all(o[3] == 0.0)
+
+
+# bf16 caches whose pieces follow the lengths: a few pairs (pieces by a cache's own length, past one group of
+# eight records), up to 128 pairs (outliers alone, or every cache where workgroups are left) and up to 255 (whole
+# caches, the longer ones in pieces), in both layouts, with empty and one-key caches
+DEALT_DECODE_CASES = [
+    # lengths, max_len, H, Hkv, head-major
+    ([16384], 16384, 8, 1, False),
+    ([20000, 0, 9000], 20480, 16, 4, True),                          # 12 pairs
+    ([16000] * 5, 16400, 8, 4, False),                               # 20 pairs: twelve pieces at most
+    ([500] * 5 + [16384] + [1, 0] + [700] * 4, 16384, 32, 4, True),  # 48 pairs, an outlier
+    ([9000 + 600 * i for i in range(12)], 16384, 32, 4, False),      # the same, none
+    ([3, 0, 16384, 2000] * 6, 16384, 8, 4, False),                   # 96 pairs: every cache
+    ([0] * 10 + [6000] + [400] * 22, 6000, 32, 4, False),            # 132 pairs
+    (list(range(100, 6100, 150)), 6100, 16, 4, False),               # 160 pairs
+    ([0] * 62 + [9000], 9000, 8, 4, True),                           # 252 pairs, one cache with keys
+    ([5200 - 20 * i for i in range(255)], 5200, 8, 1, True),         # 255 pairs of one KV head
+    ([8192], 8192, 200, 200, False),                                 # 200 KV heads of one sequence
+]
+
+
+@pytest.mark.parametrize("case", DEALT_DECODE_CASES)
+def test_decode_bf16_pieces_by_length(case):
+    lens, Lmax, H, Hkv, head_major = case
+    Bn, G = len(lens), H // Hkv
+    g = torch.Generator(device="cuda").manual_seed(81)
+    k, v = (torch.randn((Bn, Hkv, Lmax, 64) if head_major else (Bn, Lmax, Hkv, 64), generator=g,
+                        device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    if head_major:
+        k, v = k.transpose(1, 2), v.transpose(1, 2)
+    ld = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    ws = B.decode_workspace(Bn, Lmax, H)
+    ws.random_(0, 256)
+    q = torch.empty((Bn, H, 64), dtype=torch.bfloat16, device="cuda")
+    o = torch.empty_like(q)
+
+    def check(seed, call, what):
+        q.copy_(torch.randn(q.shape, generator=g.manual_seed(seed), device="cuda"))
+        o.fill_(float("nan"))
+        call()
+        ref = torch.zeros((Bn, H, 64), dtype=torch.float64, device="cuda")
+        for b in range(Bn):
+            for h in range(Hkv if lens[b] else 0):
+                rows = slice(h * G, (h + 1) * G)
+                s = q[b, rows].double() @ k[b, :lens[b], h].double().T * 0.125
+                ref[b, rows] = torch.softmax(s, 1) @ v[b, :lens[b], h].double()
+        assert_close(host(o[ld > 0]), ref[ld > 0].cpu().numpy(), BF16_TOL, f"{what} {case}")
+        assert not o[ld == 0].any()
+
+    def run():
+        B.gqa_decode(q, k, v, ld, o, scale=0.125, workspace=ws)
+
+    check(90, run, "fresh workspace")
+    check(91, run, "the same workspace")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run()
+    for n in range(3):
+        check(92 + n, graph.replay, f"replay {n}")
+        if n == 1:
+            ws.random_(0, 256)
