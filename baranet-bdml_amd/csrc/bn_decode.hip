@@ -757,7 +757,13 @@ __global__ __launch_bounds__(64 * NW) void decode_bf16_whole_kernel(DecodeParams
       const float4 r = mg.result();
       const uint32_t lo = (uint32_t)f32_to_bf16(r.x) | ((uint32_t)f32_to_bf16(r.y) << 16);
       const uint32_t hi = (uint32_t)f32_to_bf16(r.z) | ((uint32_t)f32_to_bf16(r.w) << 16);
-      *(uint2 *)(out + h * HD + d0) = make_uint2(lo, hi);
+      bf16_t *const od = out + h * HD + d0;
+      if (((uintptr_t)out & 7) == 0) {
+        *(uint2 *)od = make_uint2(lo, hi);
+      } else {  // (o is the caller's: any element may be its first)
+        od[0] = (bf16_t)lo; od[1] = (bf16_t)(lo >> 16);
+        od[2] = (bf16_t)hi; od[3] = (bf16_t)(hi >> 16);
+      }
     }
   }
 }

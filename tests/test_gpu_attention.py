@@ -890,3 +890,20 @@ def test_decode_bf16_pieces_by_length(case):
         check(92 + n, graph.replay, f"replay {n}")
         if n == 1:
             ws.random_(0, 256)
+
+
+@pytest.mark.parametrize("lens,Lmax", [([1543], 2048), ([300, 900], 1000), ([17000], 17000)])
+def test_decode_bf16_output_at_any_element(lens, Lmax):
+    # o has no alignment of its own: the merged splits' stores follow it
+    Bn, H, Hkv = len(lens), 8, 2
+    g = torch.Generator(device="cuda").manual_seed(95)
+    q, k, v = (torch.randn(s, generator=g, device="cuda", dtype=torch.bfloat16)
+               for s in ((Bn, H, 64), (Bn, Lmax, Hkv, 64), (Bn, Lmax, Hkv, 64)))
+    ld = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    want = B.gqa_decode(q, k, v, ld, scale=0.125)
+    for off in (1, 2, 3):
+        buf = torch.full((Bn * H * 64 + 8,), 7.0, dtype=torch.bfloat16, device="cuda")
+        o = buf[off:off + Bn * H * 64].view(Bn, H, 64)
+        B.gqa_decode(q, k, v, ld, o, scale=0.125)
+        assert torch.equal(o, want)
+        assert torch.all(buf[:off] == 7.0) and torch.all(buf[off + Bn * H * 64:] == 7.0)
