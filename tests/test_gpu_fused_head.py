@@ -212,3 +212,40 @@ def test_fused_head_attention_key_splits(Sq, Sk, H, Hkv, D, causal, off, alias):
     for i0 in {0, Sq - n}:
         ref = O.fused_head_attention(q[i0:i0 + n], k, v, D, H // Hkv, sc, causal, i0 + off)
         assert_close(got[i0:i0 + n], ref, FP32_TOL, f"rows {i0}..{i0 + n - 1}")
+
+
+@pytest.mark.parametrize("Sq,H,Hkv,D", [(300, 32, 4, 64), (200, 8, 8, 32), (530, 32, 4, 64)])
+def test_fused_head_attention_infinite_values_of_hidden_keys(Sq, H, Hkv, D):
+    """An infinite or NaN value reaches the rows that see its key, and no row
+    before them in their block of rows."""
+    r = np.random.default_rng(Sq)
+    q = (r.standard_normal((Sq, H * D)) * 0.3).astype(np.float32)
+    k = (r.standard_normal((Sq, Hkv * D)) * 0.3).astype(np.float32)
+    v = r.standard_normal((Sq, Hkv * D)).astype(np.float32)
+    sc = 1.0 / np.sqrt(D)
+    ref = O.fused_head_attention(q, k, v, D, H // Hkv, sc, True, 0)
+    odd = [(37, 5, np.inf), (47, 200, -np.inf), (130, 70, np.nan), (Sq - 1, 9, np.inf)]  # key, column
+    for key, col, x in odd:
+        v[key, col] = x
+    got = host(run(dev(q), dev(k), dev(v), H, Hkv, D, sc, True, 0)).reshape(Sq, Hkv, H // Hkv, D)
+    ref = ref.reshape(got.shape)
+    keep = np.ones(got.shape, bool)
+    for key, col, x in odd:
+        rows = got[key:, col // D, :, col % D]
+        assert np.isnan(rows).all() if np.isnan(x) else (rows == x).all(), (key, col)
+        keep[key:, col // D, :, col % D] = False
+    assert_close(got[keep], ref[keep], FP32_TOL, "everywhere else")
+
+
+def test_fused_head_attention_infinite_value_of_the_last_key():
+    """A ragged last tile without a mask: the last key's infinity is every row's."""
+    Sq, Sk, H, Hkv, D = 130, 300, 32, 4, 64
+    r = np.random.default_rng(3)
+    q, k = ((r.standard_normal((n, h * D)) * 0.3).astype(np.float32) for n, h in ((Sq, H), (Sk, Hkv)))
+    v = r.standard_normal((Sk, Hkv * D)).astype(np.float32)
+    ref = O.fused_head_attention(q, k, v, D, H // Hkv, 0.125, False, 0)
+    v[Sk - 1, 9] = np.inf
+    got = host(run(dev(q), dev(k), dev(v), H, Hkv, D, 0.125, False, 0))
+    cols = np.arange(H // Hkv) * D + 9
+    assert (got[:, cols] == np.inf).all()
+    assert_close(np.delete(got, cols, 1), np.delete(ref, cols, 1), FP32_TOL, "the other columns")
