@@ -223,13 +223,15 @@ __global__ __launch_bounds__(256, 2) void linear_kernel(LinParams p, RopeFreqs f
 // spread between the others, so a stage's stores, fragment reads and loads are
 // dealt evenly among its products (issued in clusters: 33.5 against 28.4 us at
 // 2048 x 2560, K 2048 without rotation; without loads and stores 22, products
-// alone 18).  Rotation angles cost one hardware sine and cosine per row and
-// frequency and tile (LDS table); per element with sincosf, and its arguments
-// read by vector loads, they took 12 of 65 us.
-// Measured (graph replay) against the 64x64-tile kernel above: 2048 x 2560, K
-// 2048 with rotation 65 -> 33.9 us (633 TFLOP/s; the library product alone 34,
-// before its separate rotation), 8192 rows 190 -> 101 (850 TFLOP/s), 512 rows
-// 25.6 -> 18.8, 64 rows 14.0 -> 11.7; 2048 x 11264 214 -> 114.  Rotating the
+// alone 18).  Rotation angles cost one sincosf per row and frequency and tile
+// (LDS table, 1.1 us of the hardware's sine and cosine, whose error after a
+// reduction to turns is 4 times as large, 1e-7 of the rotation against 2.5e-8
+// at positions 0..131071, and 8% of a sine of 1e-5); per element, with the
+// arguments read by vector loads, they took 12 of 65 us.
+// Measured (calls queued behind each other) against the 64x64-tile kernel above:
+// 2048 x 2560, K 2048 with rotation 54.0 -> 30.8 us (697 TFLOP/s), 8192 rows
+// 184.6 -> 93.5 (919 TFLOP/s), 512 rows 24.3 -> 18.8, 64 rows 13.1 -> 12.1; graph
+// replay, 2048 x 11264 214 -> 114.  Rotating the
 // tiles' first stage apart (for the memory channels) cost 5-60%.
 template <class F, int... I>
 __device__ __forceinline__ void unroll_seq(F &&f, std::integer_sequence<int, I...>) {
@@ -240,17 +242,6 @@ __device__ __forceinline__ void unroll(F &&f) {
   unroll_seq(f, std::make_integer_sequence<int, N>{});
 }
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-
-// sine and cosine of x by the hardware's, which take turns: x / 2pi split in
-// two floats, so the reduction adds no error to them
-__device__ __forceinline__ void sincos_turns(float x, float *sn, float *cs) {
-  constexpr float kHi = 0.15915493667125702f, kLo = 6.4206382e-09f;  // 1 / 2pi
-  const float hi = x * kHi;
-  const float lo = fmaf(x, kLo, fmaf(x, kHi, -hi));
-  const float t = __builtin_amdgcn_fractf(hi) + lo;
-  *sn = __builtin_amdgcn_sinf(t);
-  *cs = __builtin_amdgcn_cosf(t);
-}
 
 template <int MF, int NF, int OCC>
 __global__ __launch_bounds__(256, OCC) void linear_mn_kernel(LinParams p, RopeFreqs fr) {
@@ -428,7 +419,7 @@ __global__ __launch_bounds__(256, OCC) void linear_mn_kernel(LinParams p, RopeFr
     const int drow = 256 / hq, dq = 256 - drow * hq;
     while (row < BM) {
       float2 v;
-      sincos_turns((float)(p.pos0 + m0 + row) * fq[q], &v.x, &v.y);
+      sincosf((float)(p.pos0 + m0 + row) * fq[q], &v.x, &v.y);
       sc[row * tp + q] = v;
       row += drow;
       q += dq;
@@ -460,8 +451,8 @@ __global__ __launch_bounds__(256, OCC) void linear_mn_kernel(LinParams p, RopeFr
 #pragma unroll
       for (int i = 0; i < MF; ++i) {
         const float pos = (float)(p.pos0 + m0 + m_off + 16 * i + l16);
-        if (r0) sincos_turns(pos * fq[(gn % p.head_dim) >> 1], &ta[i].x, &ta[i].y);
-        if (r1) sincos_turns(pos * fq[((gn + 2) % p.head_dim) >> 1], &tb[i].x, &tb[i].y);
+        if (r0) sincosf(pos * fq[(gn % p.head_dim) >> 1], &ta[i].x, &ta[i].y);
+        if (r1) sincosf(pos * fq[((gn + 2) % p.head_dim) >> 1], &tb[i].x, &tb[i].y);
       }
     }
 #pragma unroll

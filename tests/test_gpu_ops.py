@@ -594,3 +594,25 @@ def test_linear_bf16_many_rows_other_layouts(form):
     y = xd if form == "in_place" else torch.empty((M, N), device="cuda", dtype=torch.bfloat16)
     B.linear_rope(xd, dev(w, torch.bfloat16), y, rope_cols=0, head_dim=64)
     assert_close(host(y), ref, BF16_TOL, form)
+
+
+@pytest.mark.parametrize("pos0", [0, 16000, 130500])
+def test_linear_rope_bf16_many_rows_rotation_alone(pos0):
+    # y is the rotation itself (x picks one row of w, whose pairs are (1, 0)): cosines and sines at bf16
+    # precision of the fp32 angle at every position, near the zeros of both (355 and 710 lie within
+    # 1e-4 of multiples of pi) as elsewhere
+    M, K, N, hd = 1024, 8, 512, 64
+    w = np.zeros((K, N), np.float32)
+    w[3, ::2] = 1.0
+    x = np.zeros((M, K), np.float32)
+    x[:, 3] = 1.0
+    y = torch.empty((M, N), device="cuda", dtype=torch.bfloat16)
+    B.linear_rope(dev(x, torch.bfloat16), dev(w, torch.bfloat16), y, rope_cols=N, position_offset=pos0, head_dim=hd)
+    base = np.array([1e4 ** float(np.float32(2 * p) / np.float32(hd)) for p in range(hd // 2)], np.float32)
+    freq = (1.0 / base.astype(np.float64)).astype(np.float32)  # op_rope.cuh:82
+    ang = ((pos0 + np.arange(M, dtype=np.float32))[:, None] * freq).astype(np.float64)
+    ref = np.stack([np.cos(ang), np.sin(ang)], -1).reshape(M, hd)
+    # half an ulp of bf16, and of fp32 sine and cosine at most four more
+    bound = (2.0 ** -8 + 2.0 ** -21) * np.abs(ref)
+    got = host(y).reshape(M, N // hd, hd)
+    assert np.all(np.abs(got - ref[:, None]) <= bound[:, None])
