@@ -1129,15 +1129,25 @@ int nt_run(const bn_view *x, const bn_view *w, const bn_view *y, int rope_cols, 
 // x 1536 7.8 / 8.4, 100 x 1536 10.2 / 8.4; K 4096, 250 x 1536 20.3 / 23.7,
 // 200 x 3072 25.0 / 26.4, 250 x 3072 26.9 / 26.6, 700 x 1536 35.3 / 30.6;
 // K 5632, 320 x 2048 27.9 / 31.7).
+// A short K leaves the loads, the epilogue and the rotation table of a large
+// tile bare (us, 64x64 tiles / here, "rot": with rotation): K 64, 800 x 2560 4.6
+// / 5.6, rot 7.2 / 10.2, 2048 x 5632 13.0 / 14.5; K 128, 800 x 2560 rot 8.0 / 10.6,
+// 100 x 2560 4.0 / 3.6, 2048 x 11264 26.0 / 27.8; K 192, 800 x 2560 rot 8.6 / 11.0,
+// 6000 x 1536 rot 21.6 / 17.3; K 256, 800 x 1536 rot (split there) 15.4 / 8.6, 800 x
+// 2560 rot 9.5 / 11.4, 800 x 5632 rot 15.7 / 14.2; K 384, 800 x 2560 rot 11.1 / 12.1;
+// K 512, the same 12.4 / 13.0, every other shape 0.29-0.99.
 // Rows that overlap, repeat or run backwards (strides below the width) stay
 // with the other kernels, whose addresses are not bounded by a descriptor over
 // whole rows; so does a y that overlaps x or w, which split-k writes only
 // after its last read.
-bool mn_takes(const bn_view *x, const bn_view *w, const bn_view *y) {
+bool mn_takes(const bn_view *x, const bn_view *w, const bn_view *y, int rope_cols) {
   constexpr int64_t kMaxRs = 1 << 21;  // 160 rows of a tile stay below 2^30 bytes
   const int m = y->h, n = w->w, k = x->w;
-  const int64_t least = 48 + (k > 2048 ? (k - 2048) / 8 : 0);
-  if (k <= 0 || m < 48 || (int64_t)m * n < 2560 * least) return false;
+  const int64_t outs = (int64_t)m * n, least = 48 + (k > 2048 ? (k - 2048) / 8 : 0);
+  const bool many = outs >= 4 << 20;
+  if (k < 128 || m < 48 || outs < 2560 * least) return false;
+  if (k < 256 && !(many ? k >= 192 : rope_cols == 0 && outs < 3 << 18)) return false;
+  if (k < 512 && rope_cols != 0 && !many && outs >= 3 << 19) return false;
   for (const bn_view *v : {x, w, y})
     if ((v->h > 1 && v->stride_h < v->w) || v->stride_h < 0 || v->stride_h >= kMaxRs) return false;
   auto apart = [](const bn_view *a, const bn_view *b) {
@@ -1365,7 +1375,7 @@ int linear_run(const bn_view *x, const bn_view *w, const bn_view *y, int rope_co
     return fail(BN_ERR_UNSUPPORTED, std::string(op) + ": problem too large");
   if ((st = ensure_device())) return st;
   hipStream_t s = as_stream(stream);
-  if (dt == BN_BF16 && epi == EPI_PLAIN && !k_dst && mn_takes(x, w, y))
+  if (dt == BN_BF16 && epi == EPI_PLAIN && !k_dst && mn_takes(x, w, y, rope_cols))
     return mn_run(x, w, y, rope_cols, position_offset, head_dim, fr, s);
   void *ws = workspace;
   bool own = false;

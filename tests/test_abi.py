@@ -485,3 +485,22 @@ def test_decode_wrappers_refuse_layouts_they_cannot_pass():
     with pytest.raises(ValueError, match="stride 1 along head_dim"):
         cols = torch.zeros((2, 16, 2, 128))[..., ::2]
         B.gqa_decode_planned(q, cols, cols, lens, [16, 16])
+
+
+def test_projection_tile_shapes_pick_every_tile():
+    """The GPU test's shapes against the cost table of bn_linear.hip: one for each
+    tile, so that a changed cost cannot drop one from the tests unnoticed."""
+    import os
+    import re
+
+    from test_gpu_ops import MANY_ROWS_TILES
+
+    src = open(os.path.join(os.path.dirname(B.__file__), "csrc", "bn_linear.hip")).read()
+    tiles = [(int(m), int(n), float(c)) for m, n, c in
+             re.findall(r"\{(\d), (\d), (\.\d+)f, linear_mn_kernel<\1, \2, \d>\}", src)]
+    assert len(tiles) == src.count("linear_mn_kernel<") and len(tiles) == 8
+    for want, (rows, k, cols, _, _, _) in MANY_ROWS_TILES.items():
+        assert k >= 512 and rows >= 48 and rows * cols >= 2560 * 48  # shapes that the kernel takes
+        cost = [-(-(-(-rows // (32 * m)) * -(-cols // (32 * n))) // 256) * c for m, n, c in tiles]
+        assert tiles[cost.index(min(cost))][:2] == want, (rows, k, cols)
+    assert set(MANY_ROWS_TILES) == {t[:2] for t in tiles}

@@ -530,24 +530,37 @@ def test_argmax_rows_ties_nan_strided():
     np.testing.assert_array_equal(host(um)[:, 0], [_argmax_sequential(row) for row in u])
 
 
-# bf16 prompts: one shape or more for every tile that the host's cost rule can pick, with ragged row and
-# column tiles, k below and past a stage of 64, positions past 4096 and head widths on both sides of
-# the rotation table's limit.
+# bf16 prompts: ragged row and column tiles, k below and past a stage of 64, positions past 4096, head widths on
+# both sides of the rotation table's limit; the short k of the first group keeps the 64 x 64-tile kernel
 MANY_ROWS_BF16 = [
     # M, K, N, rope_cols, offset, head_dim
-    (2047, 136, 2560, 2304, 0, 64),     # 128 x 160
-    (1500, 72, 2568, 2304, 4000, 64),   # 128 x 128
-    (1025, 64, 2568, 0, 0, 64),         # 128 x 96, no rotation
-    (1000, 8, 2560, 2560, 3, 128),      # 64 x 160 of less than a stage
-    (1100, 200, 2048, 1984, 7, 64),     # 64 x 128
-    (640, 2048, 2048, 2016, 100, 96),   # 64 x 96, head width no power of two
-    (330, 1992, 2568, 2304, 0, 512),    # 64 x 64, angles per element
-    (129, 520, 1024, 512, 9, 2),        # 32 x 64
-    (48, 64, 2560, 2304, 16000, 64),    # the fewest rows
+    (2047, 136, 2560, 2304, 0, 64),
+    (1500, 72, 2568, 2304, 4000, 64),
+    (1025, 64, 2568, 0, 0, 64),
+    (1000, 8, 2560, 2560, 3, 128),
+    (1100, 200, 2048, 1984, 7, 64),
+    (48, 64, 2560, 2304, 16000, 64),
+    (2047, 200, 2560, 2304, 0, 64),     # from here the large tiles: the fewest k with many outputs
+    (129, 136, 1024, 0, 0, 64),         # the fewest k without rotation
+    (48, 264, 2560, 2304, 16000, 64),   # the fewest rows; k a stage's remainder of 8
+    (640, 2048, 2048, 2016, 100, 96),   # head width no power of two
+    (330, 1992, 2568, 2304, 0, 512),    # angles per element
+    (129, 520, 1024, 512, 9, 2),
 ]
+# and a shape for every tile that the host's cost rule picks
+MANY_ROWS_TILES = {
+    (4, 5): (2047, 520, 2560, 2304, 0, 64),
+    (4, 4): (1500, 584, 2568, 2304, 4000, 64),
+    (4, 3): (1025, 512, 2568, 0, 0, 64),
+    (2, 5): (129, 576, 12296, 1024, 3, 128),
+    (2, 4): (513, 640, 3072, 1984, 7, 64),
+    (2, 3): (640, 1032, 2048, 2016, 100, 96),
+    (2, 2): (330, 1992, 2568, 2304, 0, 64),
+    (1, 2): (129, 1000, 1024, 512, 9, 2),
+}
 
 
-@pytest.mark.parametrize("case", MANY_ROWS_BF16)
+@pytest.mark.parametrize("case", MANY_ROWS_BF16 + list(MANY_ROWS_TILES.values()))
 def test_linear_rope_bf16_many_rows(case):
     M, K, N, rc, off, hd = case
     rc = rc // hd * hd
@@ -566,7 +579,7 @@ def test_linear_rope_bf16_many_rows(case):
 
 def test_linear_rope_bf16_many_rows_infinite_column():
     # an infinite column past the rotated ones leaves its neighbours as they are
-    M, K, N, rc = 512, 64, 2560, 1280
+    M, K, N, rc = 512, 512, 2560, 1280
     r = rng(67)
     x = bf16_round(np.abs(r.standard_normal((M, K))).astype(np.float32) + 0.5)
     w = bf16_round((r.standard_normal((K, N)) / np.sqrt(K)).astype(np.float32))
@@ -601,7 +614,7 @@ def test_linear_rope_bf16_many_rows_rotation_alone(pos0):
     # y is the rotation itself (x picks one row of w, whose pairs are (1, 0)): cosines and sines at bf16
     # precision of the fp32 angle at every position, near the zeros of both (355 and 710 lie within
     # 1e-4 of multiples of pi) as elsewhere
-    M, K, N, hd = 1024, 8, 512, 64
+    M, K, N, hd = 1024, 256, 512, 64
     w = np.zeros((K, N), np.float32)
     w[3, ::2] = 1.0
     x = np.zeros((M, K), np.float32)
