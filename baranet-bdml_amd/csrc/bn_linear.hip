@@ -223,14 +223,14 @@ __global__ __launch_bounds__(256, 2) void linear_kernel(LinParams p, RopeFreqs f
 // spread between the others, so a stage's stores, fragment reads and loads are
 // dealt evenly among its products (issued in clusters: 33.5 against 28.4 us at
 // 2048 x 2560, K 2048 without rotation; without loads and stores 22, products
-// alone 18).  Rotation angles cost one sincosf per row and frequency and tile
-// (LDS table, 1.1 us of the hardware's sine and cosine, whose error after a
-// reduction to turns is 4 times as large, 1e-7 of the rotation against 2.5e-8
-// at positions 0..131071, and 8% of a sine of 1e-5); per element, with the
-// arguments read by vector loads, they took 12 of 65 us.
+// alone 18).  Rotation angles cost one sine and cosine per row and frequency and
+// tile (LDS table), of fp32 precision: with sincosf and an index that wraps, 30.7
+// against 29.4 us at 2048 x 2560; the hardware's, which take turns, no less than
+// 29.5 and four times the error (8% of a sine of 1e-5).  Per element with
+// sincosf, its arguments read by vector loads, they took 12 of 65 us.
 // Measured (calls queued behind each other) against the 64x64-tile kernel above:
-// 2048 x 2560, K 2048 with rotation 54.0 -> 30.8 us (697 TFLOP/s), 8192 rows
-// 184.6 -> 93.5 (919 TFLOP/s), 512 rows 24.3 -> 18.8, 64 rows 13.1 -> 12.1; graph
+// 2048 x 2560, K 2048 with rotation 54.0 -> 29.4 us (730 TFLOP/s), 8192 rows
+// 184.6 -> 90.8 (946 TFLOP/s), 512 rows 24.3 -> 18.3, 64 rows 13.1 -> 11.7; graph
 // replay, 2048 x 11264 214 -> 114.  Rotating the
 // tiles' first stage apart (for the memory channels) cost 5-60%.
 template <class F, int... I>
@@ -242,6 +242,34 @@ __device__ __forceinline__ void unroll(F &&f) {
   unroll_seq(f, std::make_integer_sequence<int, N>{});
 }
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+// sine and cosine of x: Cody and Waite's reduction by a multiple k of pi/2 in
+// three floats (the first difference is exact by cancellation, the others add
+// half an ulp of the remainder r) and the Taylor series of both on [-pi/4, pi/4]
+// (first terms left out below 1.8e-9).  Past 2^17 the library's.  Error over
+// positions 0..131071 and 32 frequencies against 64 bits 2.40e-8 (2-norm), at most
+// 1.45 ulp; sincosf's, the other kernels', 2.55e-8 and 1.57.
+__device__ __forceinline__ void angle_sincos(float x, float *sn, float *cs) {
+  const float k = rintf(x * 0.63661977f);
+  float r = fmaf(k, -1.57079637f, x);
+  r = fmaf(k, 4.37113883e-08f, r);
+  r = fmaf(k, 1.71512451e-15f, r);
+  const float z = r * r;
+  float s = fmaf(z, 2.75573192e-06f, -1.98412698e-04f);
+  s = fmaf(z, s, 8.33333333e-03f);
+  s = fmaf(z, s, -1.66666667e-01f);
+  s = fmaf(r * z, s, r);
+  float c = fmaf(z, -2.75573192e-07f, 2.48015873e-05f);
+  c = fmaf(z, c, -1.38888889e-03f);
+  c = fmaf(z, c, 4.16666667e-02f);
+  c = fmaf(z, c, -0.5f);
+  c = fmaf(z, c, 1.0f);
+  const int q = (int)k;
+  const float a = q & 1 ? c : s, b = q & 1 ? s : c;
+  *sn = __uint_as_float(__float_as_uint(a) ^ ((uint32_t)(q & 2) << 30));
+  *cs = __uint_as_float(__float_as_uint(b) ^ ((uint32_t)((q + 1) & 2) << 30));
+  if (!(fabsf(x) < 131072.f)) sincosf(x, sn, cs);
+}
 
 template <int MF, int NF, int OCC>
 __global__ __launch_bounds__(256, OCC) void linear_mn_kernel(LinParams p, RopeFreqs fr) {
@@ -415,17 +443,27 @@ __global__ __launch_bounds__(256, OCC) void linear_mn_kernel(LinParams p, RopeFr
   float2 *const sc = reinterpret_cast<float2 *>(smem);
   if (table) {
     __syncthreads();  // the last stage's reads ahead
-    int row = tid / hq, q = tid - row * hq;
-    const int drow = 256 / hq, dq = 256 - drow * hq;
-    while (row < BM) {
-      float2 v;
-      sincosf((float)(p.pos0 + m0 + row) * fq[q], &v.x, &v.y);
-      sc[row * tp + q] = v;
-      row += drow;
-      q += dq;
-      if (q >= hq) {
-        q -= hq;
-        ++row;
+    if (256 % hq == 0) {  // a thread's frequency is one
+      const int drow = 256 / hq, row0 = tid / hq, q = tid - row0 * hq;
+      const float f = fq[q];
+      for (int row = row0; row < BM; row += drow) {
+        float2 v;
+        angle_sincos((float)(p.pos0 + m0 + row) * f, &v.x, &v.y);
+        sc[row * tp + q] = v;
+      }
+    } else {
+      int row = tid / hq, q = tid - row * hq;
+      const int drow = 256 / hq, dq = 256 - drow * hq;
+      while (row < BM) {
+        float2 v;
+        angle_sincos((float)(p.pos0 + m0 + row) * fq[q], &v.x, &v.y);
+        sc[row * tp + q] = v;
+        row += drow;
+        q += dq;
+        if (q >= hq) {
+          q -= hq;
+          ++row;
+        }
       }
     }
     __syncthreads();
@@ -451,8 +489,8 @@ __global__ __launch_bounds__(256, OCC) void linear_mn_kernel(LinParams p, RopeFr
 #pragma unroll
       for (int i = 0; i < MF; ++i) {
         const float pos = (float)(p.pos0 + m0 + m_off + 16 * i + l16);
-        if (r0) sincosf(pos * fq[(gn % p.head_dim) >> 1], &ta[i].x, &ta[i].y);
-        if (r1) sincosf(pos * fq[((gn + 2) % p.head_dim) >> 1], &tb[i].x, &tb[i].y);
+        if (r0) angle_sincos(pos * fq[(gn % p.head_dim) >> 1], &ta[i].x, &ta[i].y);
+        if (r1) angle_sincos(pos * fq[((gn + 2) % p.head_dim) >> 1], &tb[i].x, &tb[i].y);
       }
     }
 #pragma unroll

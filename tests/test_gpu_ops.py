@@ -609,12 +609,12 @@ def test_linear_bf16_many_rows_other_layouts(form):
     assert_close(host(y), ref, BF16_TOL, form)
 
 
-@pytest.mark.parametrize("pos0", [0, 16000, 130500])
-def test_linear_rope_bf16_many_rows_rotation_alone(pos0):
+@pytest.mark.parametrize("pos0,hd", [(0, 64), (16000, 64), (130500, 64), (0, 96), (300, 512), (-900, 64)])
+def test_linear_rope_bf16_many_rows_rotation_alone(pos0, hd):
     # y is the rotation itself (x picks one row of w, whose pairs are (1, 0)): cosines and sines at bf16
     # precision of the fp32 angle at every position, near the zeros of both (355 and 710 lie within
-    # 1e-4 of multiples of pi) as elsewhere
-    M, K, N, hd = 1024, 256, 512, 64
+    # 1e-4 of multiples of pi) as elsewhere; past 2^17; a table whose threads change their frequency, none
+    M, K, N = 1024, 256, -(-512 // hd) * hd
     w = np.zeros((K, N), np.float32)
     w[3, ::2] = 1.0
     x = np.zeros((M, K), np.float32)
