@@ -1201,7 +1201,12 @@ __global__ __launch_bounds__(64 * KW, 2) void prefill_f32_ks_kernel(PrefillParam
 // Groups that are no multiple of 4 have no shared form; there the row kernel
 // (one head per workgroup) holds above 1024 units (8 heads, B=4 S=2048: 34.2
 // against s4 39.4; S=4096 52.8 against 36.5), or 512 even ones (B=2 S=2048
-// without mask 27.9 against 32.2; B=1 27.0 against 18.7).
+// without mask 27.9 against 32.2; B=1 27.0 against 18.7), and a few tiles' keys
+// dealt to four waves cost more than they save (ratio to the row kernel, one
+// tile: 16 units 1.04, 640 1.21; two: 256 0.93, 320 1.12, 960 1.29; three: 384
+// 0.98, 600 1.10; four: 512 0.90, 800 1.17; ten: 720 0.92, 800 1.05, 960 1.08).
+// Groups of 4: one or two tiles, 256 units 0.85-0.9, 320-576 1.05-1.17; three, 528
+// 1.13; the shared form from 640 units 0.97.
 // fp32 (matrix-core time alone counts): rows/s8/s4/two waves S=512 44.9/21.0/
 // 19.6/30.4, B=4 S=512 60.6/72.4/56.1/50.2, S=2048 211/171/148/160, B=2 S=2048
 // 311/339/286/281 and without mask 567/582/531/572.  Rows of more than 2560
@@ -1221,7 +1226,11 @@ KsKind ks_kind(int dtype, int batch, int n_kv_heads, int group, int seq_q, int s
     if (first + 32 * nt > 2 * 2560 + 32 || (!causal && units >= 4096)) return KsKind::none;
     return units <= (nt >= 64 ? 2048 : 1536) ? few : KsKind::split2;
   }
-  if (group % 4 != 0) return units > (even ? 512 : 1024) ? KsKind::none : few;
+  if (group % 4 != 0) {
+    const int64_t most = nt <= 1 ? 0 : nt == 2 ? 256 : nt == 3 ? 448 : nt <= 6 ? 640 : nt <= 11 ? 768 : 1024;
+    return units > (even ? std::min<int64_t>(most, 512) : most) ? KsKind::none : few;
+  }
+  if (group % 8 != 0 && nt <= 3 && units > (nt == 3 ? 448 : 256) && units < 640) return KsKind::none;
   const bool wide = group >= 8;
   if (units < (even ? 768 : nt <= 16 ? 640 : 1024)) return few;
   if (nt <= 4) return KsKind::shared;

@@ -658,8 +658,12 @@ SPLIT_CASES = [
     ("bf16", 1, 33, 1057, 8, 1, 1, 1024),    # eight key parts, one (batch, KV head)
     ("bf16", 1, 1, 1025, 2, 2, 1, 1024),     # more waves than the last round has tiles
     ("bf16", 3, 31, 95, 6, 2, 1, 64),        # four key parts, six (batch, KV head)s
-    ("bf16", 1, 65, 3, 4, 4, 0, 0),          # fewer keys than a tile, no mask
-    ("bf16", 2, 40, 70, 10, 2, 1, -9),       # rows that see no key, group of 5
+    ("bf16", 1, 65, 3, 4, 4, 0, 0),          # fewer keys than a tile, no mask: the row kernel
+    ("bf16", 1, 65, 3, 8, 1, 0, 0),          # the same in a group of 8: four key parts
+    ("bf16", 2, 40, 70, 10, 2, 1, -9),       # rows that see no key, one tile, group of 5: the row kernel
+    ("bf16", 2, 40, 70, 16, 2, 1, -9),       # the same, group of 8
+    ("bf16", 2, 90, 120, 10, 2, 1, -9),      # rows that see no key, group of 5
+    ("bf16", 9, 37, 37, 16, 4, 1, 0),        # group of 4, two tiles: the row kernel
     ("bf16", 8, 97, 97, 32, 4, 1, 0),        # shared tiles, two key parts
     ("bf16", 3, 352, 400, 32, 4, 1, 48),     # the same, 12 (batch, KV head)s
     ("bf16", 24, 97, 129, 32, 4, 1, 32),     # shared tiles, one key part
