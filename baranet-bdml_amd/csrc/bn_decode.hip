@@ -1283,8 +1283,10 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(DecodeParams p) {
   Elem<T>::store(out + 3, r.w);
 }
 
-// workgroup targets of the fp32 chunks, and of the four-KV-head bf16 chunks
-// that the no-allocation call's size limit is stated in
+// workgroup targets of the fp32 chunks, and of the chunks of four KV heads in
+// which the no-allocation call counts a bf16 call's size: its limit is the
+// caller's to rely on, so it does not follow the pieces, which need less
+// (17.3 MB at most of the 32)
 constexpr int kMinWg = 2048, kRowsMinWg = 512;
 int choose_chunk(int batch, int max_len, int units, int min_wg) {
   // enough workgroups to cover the 256 CUs several times over (a partial last

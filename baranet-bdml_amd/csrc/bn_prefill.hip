@@ -613,11 +613,14 @@ __device__ __forceinline__ bool decode_work_units(const PrefillParams &p, int n_
 // kernel above in this split measured the same at HW > 1 and slower at HW == 1
 // (182 VGPRs; B=1 S=2048 43 against 37 us), two tiles of loads in flight
 // changed nothing.  Against the row kernel, which gives these calls 32-256
-// workgroups that walk every key alone: 256 rows behind 4096 cached 74 -> 21
-// us, 64 rows of 4160 keys 71 -> 18, S=512 15.9 -> 7.7, B=2 S=777 21.7 -> 15.5,
-// S=2048 40.3 -> 28.7.  HW == 1 is bound by the CU's L1 and LDS ports (every
-// unit pulls its own 8 KB per tile through both), HW == 4 by the softmax's
-// VALU work beside the products.
+// workgroups that walk every key alone: 256 rows behind 4096 cached 74.2 -> 20.2
+// us, 64 rows of 4160 keys 70.1 -> 17.4, S=512 15.3 -> 7.3, B=2 S=777 20.1 -> 14.3,
+// S=2048 40.5 -> 28.8 (calls queued behind each other).  HW == 1 is bound by
+// the CU's LDS and L1 ports, through both of which every unit pulls its own 8 KB
+// per tile (counters, 256 rows behind 4096, share of the busy CU's cycles: LDS 89%,
+// L1 accesses 49%, VALU 31%, matrix cores 24%); HW == 4 by no one of them (B=2
+// S=777: LDS and VALU 43% each, matrix cores 23%) but by latency: its waves wait
+// 44% of their time for memory or LDS.
 // Waves without a tile, and rows that see no key, keep m = -inf and weigh 0.
 template <int HW, int KW, int OCC>
 __global__ __launch_bounds__(64 * HW * KW, OCC) void prefill_bf16_ks_kernel(PrefillParams p) {
@@ -995,17 +998,19 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillParams p) {
 // --------------------------------------------------------- fp32, keys split
 // The same split on v_mfma_f32_32x32x2f32 (64 cycles each: 64 of them per
 // 32-key tile and unit, so matrix-core time is all that counts and one wave
-// walking a 512-key row takes 27 of the row kernel's 43 us).  One (head, 32 query rows) unit per workgroup, its tiles dealt to KW
-// waves, no barrier before the merge: a wave stages its own K tile in LDS
+// walking a 512-key row takes 27 of the row kernel's 43 us; counters at S=512:
+// matrix cores 50% of the busy CU's cycles, VALU 15%, LDS 15%, the rest units of
+// unequal length).  One (head, 32 query rows) unit per workgroup, its tiles dealt
+// to KW waves, no barrier before the merge: a wave stages its own K tile in LDS
 // (rows of 272 B) one tile ahead and reads V straight from memory -- P^T is
 // the PV product's B operand as the scores left it, so an A operand is two
 // adjacent d of one key row per lane, 256 contiguous bytes per half-wave --
 // with the loads issued before the tile's 32 score products, which cover
 // them.  Exact online softmax per tile.
-// Measured (graph replay, against 4 waves x 32 rows over shared 64-key
-// blocks): B=1 S=512 H=32 44.9 -> 17.2 us, S=2048 211 -> 148, B=4 S=2048 596
-// -> 544 (126 TFLOP/s, 82% of what a large fp32 product reaches), 256 rows
-// behind 4096 333 -> 76.
+// Measured (calls queued behind each other, against 4 waves x 32 rows over
+// shared 64-key blocks): B=1 S=512 H=32 43.7 -> 17.1 us, S=2048 213 -> 154, B=4
+// S=2048 598 -> 560 (kernel trace 549: 125 TFLOP/s, 82% of what a large fp32
+// product reaches), 256 rows behind 2000 176 -> 47.
 template <int KW>
 __global__ __launch_bounds__(64 * KW, 2) void prefill_f32_ks_kernel(PrefillParams p) {
   constexpr int KP = HD + 4;  // K row and O row pitch, floats
@@ -1209,10 +1214,14 @@ __global__ __launch_bounds__(64 * KW, 2) void prefill_f32_ks_kernel(PrefillParam
 // 1.13; the shared form from 640 units 0.97.
 // fp32 (matrix-core time alone counts): rows/s8/s4/two waves S=512 44.9/21.0/
 // 19.6/30.4, B=4 S=512 60.6/72.4/56.1/50.2, S=2048 211/171/148/160, B=2 S=2048
-// 311/339/286/281 and without mask 567/582/531/572.  Rows of more than 2560
-// keys on average keep the row kernel's order of sums: the split's differs from
-// it by 1.1e-6 (relative, over the output) at 2000 keys and by 2.1e-6 at 4352
-// (it is the nearer one to 64 bits, 1.1e-6 against 2.4e-6).
+// 311/339/286/281 and without mask 567/582/531/572 (the choice there is between
+// rows and two waves: four were measured at this size alone).  The line at
+// 2560 keys a row on average is not one of speed or of precision, both of which
+// the split has on its side past it too (256 rows behind 4096 333 -> 76 us,
+// error against 64 bits 2.4e-6 -> 1.1e-6): a call that has been answered keeps its
+// answer to 2e-6, which is what fp32 outputs are held to from one build to the
+// next, and the two orders of sums differ by 1.1e-6 (relative, over the output)
+// at 2000 keys and by 2.1e-6 at 4352.
 enum class KsKind { none, shared, shared2, split2, split4, split8 };
 KsKind ks_kind(int dtype, int batch, int n_kv_heads, int group, int seq_q, int seq_kv, int causal,
                int seq_offset) {

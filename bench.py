@@ -538,9 +538,9 @@ def bench_fused_head_kernel(steps, warmup, S=128):
 
 def bench_fused_head_long(steps, warmup, sizes=(512, 2048)):
     """bn_fused_head_attention on longer prompts (32/4 heads, head_dim 64,
-    fp32, causal), where it runs on the matrix cores: group sums of Q, 32 x
-    128 score blocks on v_mfma_f32_32x32x2f32, a log-sum-exp merge (three
-    launches and a pool allocation per call).  Eager launches back to back,
+    fp32, causal), where it runs on the matrix cores: 16-row blocks with the
+    keys split over waves and workgroups on v_mfma_f32_16x16x4f32, and a
+    log-sum-exp merge (two launches per call).  Eager launches back to back,
     events on the stream; the work counted is the causal half of the two
     products at the group-summed width (2 x 2 x 256 flops per visible pair)."""
     import torch
@@ -558,8 +558,8 @@ def bench_fused_head_long(steps, warmup, sizes=(512, 2048)):
         tf = flop / (ms * 1e-3) / 1e12
         res[f"S{S}"] = {"us_per_call": round(ms * 1e3, 2), "flop": flop,
                         "roofline": roofline("mfma", tf, PEAK_FP32_TFLOPS, "TFLOP/s")}
-    res["note"] = ("eager calls (host launch of three kernels and a pool round trip per call: "
-                   "host-bound at 512 rows); device times per kernel in the rocprofv3 summary")
+    res["note"] = ("eager calls (host launch of two kernels per call); device times per kernel in "
+                   "the rocprofv3 summary")
     return res
 
 

@@ -428,7 +428,8 @@ int bn_gqa_decode_planned_strided(int dtype, const void *q, const void *k_cache,
  * the process ends; its address is looked up once per device by bn_init).
  * It calls no hipMalloc, hipFree or pool allocation; a call whose partials
  * would exceed the array fails with BN_ERR_UNSUPPORTED before any device
- * work.  Every call on one GPU shares that GPU's array and leaves its last
+ * work (counted in chunks of 128 to 1024 keys for either type, also where bf16
+ * caches are cut into fewer pieces).  Every call on one GPU shares that GPU's array and leaves its last
  * contents there (nothing needs clearing: each call writes every record it
  * reads; the short-cache split's counters return to zero at the end of each
  * launch), so calls that overlap on one GPU -- on different streams, or from

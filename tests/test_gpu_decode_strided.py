@@ -67,8 +67,8 @@ CASES = [
     ("bf16", 80, 300, 16, 4, "ragged"),    # the same kernel, G = 4, short caches
     ("bf16", 512, 96, 16, 2, "ragged"),    # the same kernel, the largest batch that sums its lengths
     ("bf16", 520, 96, 16, 2, "ragged"),    # past it: four waves for every cache, any layout
-    ("bf16", 2, 4096, 32, 4, "ragged"),    # split-K, whole-row kernel (4 KV heads per workgroup)
-    ("bf16", 3, 1000, 16, 2, "ragged"),    # split-K, per-head kernel (n_kv_heads not a multiple of 4)
+    ("bf16", 2, 4096, 32, 4, "ragged"),    # split over workgroups, 4 KV heads
+    ("bf16", 3, 1000, 16, 2, "ragged"),    # split over workgroups, n_kv_heads not a multiple of 4
     ("f32", 2, 2048, 32, 4, "ragged"),     # fp32 split-K
     ("f32", 1, 640, 32, 4, "uniform"),     # fp32 short-cache split, merged in the launch
     ("f32", 3, 300, 8, 2, "ragged"),

@@ -58,7 +58,7 @@ def run_noalloc(dtype, qd, kd, vd, ld, o):
 
 # (dtype, H, Hkv, first call (B, L, lens), second call (B, L, lens)); the
 # second call is smaller in batch and cache length
-PATHS = {
+PATHS = {  # (bf16 splits: 4 KV heads, 2 KV heads)
     "bf16_rows_split": ("bf16", 32, 4, (6, 3000, [3000, 1, 2047, 129, 3000, 700]),
                         (3, 1000, [1000, 300, 5])),
     "bf16_head_split": ("bf16", 16, 2, (5, 2500, [2500, 17, 1024, 2000, 64]),
