@@ -223,7 +223,8 @@ __global__ __launch_bounds__(256, 2) void linear_kernel(LinParams p, RopeFreqs f
 // spread between the others, so a stage's stores, fragment reads and loads are
 // dealt evenly among its products (issued in clusters: 33.5 against 28.4 us at
 // 2048 x 2560, K 2048 without rotation; without loads and stores 22, products
-// alone 18).  Rotation angles cost one sine and cosine per row and frequency and
+// alone 18; counters of that shape with rotation, share of the busy CU's
+// cycles: LDS 60% and bank conflicts 15%, matrix cores 29%).  Rotation angles cost one sine and cosine per row and frequency and
 // tile (LDS table), of fp32 precision: with sincosf and an index that wraps, 30.7
 // against 29.4 us at 2048 x 2560; the hardware's, which take turns, no less than
 // 29.5 and four times the error (8% of a sine of 1e-5).  Per element with
