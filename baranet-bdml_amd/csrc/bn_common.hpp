@@ -154,6 +154,18 @@ struct DecMerge {
       }
     }
   }
+  // the same by an address per record, past the caches
+  template <class F>
+  __device__ __forceinline__ void load8_from(F &&rec, int n, int s0, int d0) {
+    auto rd = [](const float *a) { return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); };
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float *ps = rec(min(s0 + j, n - 1));
+      ms[j] = rd(ps);
+      ls[j] = rd(ps + 1);
+      as[j] = make_float4(rd(ps + 2 + d0), rd(ps + 3 + d0), rd(ps + 4 + d0), rd(ps + 5 + d0));
+    }
+  }
   // the same values in two parts: acc from the records, (m, l) from a table
   // of pairs (stride 2 floats; e.g. gathered into LDS)
   __device__ __forceinline__ void load_acc8(const float *part, int n_split, int s0, int d0) {

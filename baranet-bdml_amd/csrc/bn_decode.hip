@@ -82,16 +82,16 @@ __device__ __forceinline__ float row_sum(float x) {
   return x;
 }
 
-// Sum over the wave, a uniform value, without an LDS round trip: DPP moves inside
-// each 16-lane row, then the rows' sums by readlane.
+// Largest of the wave's values (not negative), uniform, without an LDS round
+// trip: DPP moves inside each 16-lane row, then the rows' by readlane.
 template <int CTRL>
-__device__ __forceinline__ int dpp_add(int v) {
-  return v + __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, false);
+__device__ __forceinline__ int dpp_max(int v) {
+  return max(v, __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, false));
 }
-__device__ __forceinline__ int wave_sum_i32(int v) {
-  v = dpp_add<0x140>(dpp_add<0x141>(dpp_add<0x4E>(dpp_add<0xB1>(v))));
-  return __builtin_amdgcn_readlane(v, 0) + __builtin_amdgcn_readlane(v, 16) + __builtin_amdgcn_readlane(v, 32) +
-         __builtin_amdgcn_readlane(v, 48);
+__device__ __forceinline__ int wave_max_i32(int v) {
+  v = dpp_max<0x140>(dpp_max<0x141>(dpp_max<0x4E>(dpp_max<0xB1>(v))));
+  return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+             max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
 }
 
 struct DecodeParams {
@@ -100,10 +100,8 @@ struct DecodeParams {
   void *o;
   float *ws;  // partials: [batch*n_heads][n_split][HD + 2]
   int batch, max_len, n_heads, n_kv_heads, n_split, chunk;
-  // dealt caches: pieces of a cache at least (n_split: at most), the workgroups
-  // per KV head for further pieces, and whether only far longer caches than the
-  // others get them
-  int min_split = 1, more = 0, outliers = 0;
+  int min_split = 1;  // pieces of a cache at least (n_split: at most)
+  int groups = 0;     // dealt batches: workgroups per KV head (0: pieces per cache)
   float c;        // scale * log2(e)
   int hlen = -1;  // >= 0: every sequence's length, from the host (lens not read)
   // cache strides in elements: sequence, KV head, key row (a contiguous
@@ -409,12 +407,12 @@ constexpr int WKP = HD + 8;  // tile row pitch, 144 B: b128 K reads of 16 rows a
 
 // a cache up to this length is one split's (500 keys: 5.8 us, in 2-8 splits 6.9)
 constexpr int kSplitMinLen = 512;
-// how a cache is dealt to workgroups: whole, in n_split equal pieces, or in
-// pieces that follow its length and the batch's
-constexpr int kWhole = 0, kSplit = 1, kDealt = 2;
-constexpr int kPieceMinLen = 1024;  // keys of a dealt piece at least
-constexpr int kFewPairs = 32;       // below, a cache's pieces follow its own length alone
-constexpr int kDealtMax = 256;      // sequences of a dealt batch (4 a lane)
+// how caches are dealt to workgroups: whole, each in up to n_split equal pieces,
+// in pieces by its own length, or the batch in equal shares
+constexpr int kWhole = 0, kSplit = 1, kByLength = 2, kDealt = 3;
+constexpr int kPieceMinLen = 1024;  // keys of each piece of a cache in more than min_split
+constexpr int kShareMin = 8;        // tiles of a share at least
+constexpr int kUneven = 40;         // tiles over a share that the longest cache's piece may have
 constexpr unsigned long long kArrive = 0x5bd1e995a93c71d4ull;
 // keys per split of a cache: whole rounds of the workgroup's four tiles
 template <int NW>
@@ -425,11 +423,13 @@ __device__ __forceinline__ int split_chunk(int len, int n_split) {
 }
 
 // NW waves per workgroup: WWV, or WWX with the long-cache adaptation.
-// SPLIT (fewer (sequence, KV head) pairs than compute units; kSplit equal
-// pieces, kDealt by the lengths, dealt_splits): up to n_split
-// workgroups per pair, each over a run of the cache, so that a few caches
-// have most of their loads in flight at once; bound by latencies (launch, one
-// or two memory round trips, the merge).  A split writes its merged (m, l,
+// SPLIT (fewer (sequence, KV head) pairs than compute units): a cache in pieces,
+// so that a few caches have most of their loads in flight at once; bound by
+// latencies (launch, one or two memory round trips, the merge).  kSplit, kByLength:
+// up to n_split workgroups per pair, each over a run of the cache.  kDealt: the
+// sequences' tiles in a row, an equal share of it per workgroup, which takes the
+// caches in it one after another, so that long and uneven batches end together
+// (dealt_groups).  A split writes its merged (m, l,
 // acc) record through to memory, waits for it, and counts itself in on the
 // pair's arrival word; the last one to arrive merges the records and writes
 // the output, in the same launch.  Measured (graph replay, B=1 / 4 KV heads, G
@@ -462,308 +462,332 @@ __global__ __launch_bounds__(64 * NW) void decode_bf16_whole_kernel(DecodeParams
   const int l16 = lane & 15, grp = lane >> 4;
   // the KV heads of a sequence's (split's) rows next to each other
   const int g = blockIdx.x % p.n_kv_heads, bs = blockIdx.x / p.n_kv_heads;
-  int b = SPLIT ? bs / p.n_split : bs, split = SPLIT ? bs - b * p.n_split : 0;
   auto clamp_len = [&](int x) { return x < 0 ? 0 : (x > p.max_len ? p.max_len : x); };
 
-  // the batch's total length (batches up to kMeanBatchMax sequences), summed
-  // by every wave itself (no barrier), read with this sequence's length
-  const bool adapt = !SPLIT && NW > WWV && p.batch <= kMeanBatchMax;
-  int part = 0;
-  if (adapt)
-    for (int i = lane; i < p.batch; i += 64) part += clamp_len(p.lens[i]);
-  int pieces = SPLIT ? p.n_split : 1;
-  if (DEAL == kDealt && p.batch * p.n_kv_heads >= kFewPairs) {
-    // min_split pieces of every cache first; the p.more workgroups per
-    // KV head after those take the further pieces of the longer caches, found by
-    // a scan over the batch that every wave makes for itself (lane: 4 sequences)
-    int t[4], sum = 0;
+  // One piece: keys [k0, kw1) of sequence b, by nw waves; piece q of the
+  // pieces() that hold the cache's keys (a division, left until the loads are
+  // through).  bin0: the group of a dealt cache's first piece.
+  auto run = [&](const int b, const int k0, const int kw1, const int nw, auto pieces, const int q,
+                 const int bin0) __attribute__((always_inline)) {
+    bf16_t *const out = (bf16_t *)p.o + ((int64_t)b * p.n_heads + (int64_t)g * G) * HD;
+    // wave w < nw takes the 32-key tiles w, w + nw, w + 2*nw, ...: the waves of
+    // a workgroup stream adjacent tiles (a contiguous key range per wave, or the
+    // KV heads of one sequence placed on one XCD, measured 3-4% slower)
+    const int all_tiles = (kw1 - k0 + TK - 1) / TK;
+    const int kw0 = k0 + TK * wave;
+    const int tstride = TK * nw;  // keys between a wave's tiles
+    const int ntiles = wave < nw && all_tiles > wave ? (all_tiles - wave + nw - 1) / nw : 0;
+
+    const int64_t kv_rs = p.kv_rs;
+    const bf16_t *Kr = (const bf16_t *)p.k + b * p.kv_bs + g * p.kv_hs;
+    const bf16_t *Vr = (const bf16_t *)p.v + b * p.kv_bs + g * p.kv_hs;
+
+    dbf16x8_t qb[2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int s = 4 * lane + i;
-      t[i] = s < p.batch ? min((clamp_len(p.lens[s]) + TK - 1) / TK, 1 << 22) : 0;
-      sum += t[i];
+    for (int t = 0; t < 2; ++t) {
+      if (l16 < G)
+        qb[t] = *(const dbf16x8_t *)((const bf16_t *)p.q +
+                                     ((int64_t)b * p.n_heads + g * G + l16) * HD + 8 * grp + 32 * t);
+      else
+        qb[t] = dbf16x8_t{};
     }
-    const int total = wave_sum_i32(sum);  // <= 2^30
-    // A cache has as many pieces as it holds whole shares.  A share is more
-    // than the batch's tiles over p.more, so the caches hold fewer of them than
-    // there are workgroups.
-    const int share = max((int)((uint32_t)total / (uint32_t)p.more) + 1, kPieceMinLen / TK);
-    auto pieces_of = [&](int tiles) {
-      if (p.outliers && (int64_t)tiles * p.batch <= 4 * (int64_t)total) return p.min_split;
-      return min(max((int)((uint32_t)tiles / (uint32_t)share), p.min_split), p.n_split);
+
+    // lane's 16-byte chunks of a tile: rows crow + 8i (i = 0..3), columns ccol..ccol+7
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    struct RegTile {
+      u32x4 k0, k1, k2, k3, v0, v1, v2, v3;
     };
-    const int j = bs - p.batch * p.min_split;
-    if (j < 0) {
-      b = bs / p.min_split;
-      split = bs - b * p.min_split;
-    } else {
-      int more[4], in = 0;
+    const int crow = lane >> 3, ccol = (lane & 7) * 8;
+    auto gload = [&](RegTile &r, int ti) __attribute__((always_inline)) {
+      const int kb = kw0 + tstride * min(ti, ntiles - 1);  // clamped: same load count on every path
+      const int last = min(kb + TK, kw1) - 1;  // past the end: a valid row, masked to P = 0
+      const int64_t o0 = (int64_t)min(kb + crow, last) * kv_rs + ccol;
+      const int64_t o1 = (int64_t)min(kb + crow + 8, last) * kv_rs + ccol;
+      const int64_t o2 = (int64_t)min(kb + crow + 16, last) * kv_rs + ccol;
+      const int64_t o3 = (int64_t)min(kb + crow + 24, last) * kv_rs + ccol;
+      // streamed once: non-temporal loads
+      r.k0 = __builtin_nontemporal_load((const u32x4 *)(Kr + o0)); r.v0 = __builtin_nontemporal_load((const u32x4 *)(Vr + o0));
+      r.k1 = __builtin_nontemporal_load((const u32x4 *)(Kr + o1)); r.v1 = __builtin_nontemporal_load((const u32x4 *)(Vr + o1));
+      r.k2 = __builtin_nontemporal_load((const u32x4 *)(Kr + o2)); r.v2 = __builtin_nontemporal_load((const u32x4 *)(Vr + o2));
+      r.k3 = __builtin_nontemporal_load((const u32x4 *)(Kr + o3)); r.v3 = __builtin_nontemporal_load((const u32x4 *)(Vr + o3));
+    };
+    bf16_t *const kt = KT[wave], *const vt = VT[wave];
+    auto lstore = [&](const RegTile &r) __attribute__((always_inline)) {
+      *(u32x4 *)(kt + crow * WKP + ccol) = r.k0;
+      *(u32x4 *)(kt + (crow + 8) * WKP + ccol) = r.k1;
+      *(u32x4 *)(kt + (crow + 16) * WKP + ccol) = r.k2;
+      *(u32x4 *)(kt + (crow + 24) * WKP + ccol) = r.k3;
+      *(u32x4 *)(vt + crow * WKP + ccol) = r.v0;
+      *(u32x4 *)(vt + (crow + 8) * WKP + ccol) = r.v1;
+      *(u32x4 *)(vt + (crow + 16) * WKP + ccol) = r.v2;
+      *(u32x4 *)(vt + (crow + 24) * WKP + ccol) = r.v3;
+    };
+
+    float m = -INFINITY, l = 0.f;
+    df32x4_t o[4] = {df32x4_t{}, df32x4_t{}, df32x4_t{}, df32x4_t{}};
+    const float c = p.c;
+    // one 32-key tile from this wave's LDS tile; keys kb .. kb + 31
+    auto compute = [&](int kb) __attribute__((always_inline)) {
+      const bf16_t *kl = kt + 8 * grp;
+      df32x4_t s[2];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        more[i] = pieces_of(t[i]) - p.min_split;
-        in += more[i];
+      for (int u = 0; u < 2; ++u) {
+        const bf16_t *kp = kl + (16 * u + l16) * WKP;
+        s[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const dbf16x8_t *)(kp), qb[0], df32x4_t{},
+                                                       0, 0, 0);
+        s[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const dbf16x8_t *)(kp + 32), qb[1], s[u],
+                                                       0, 0, 0);
       }
-      const int own = in;
+      // s[u][i] = score of key kb + 16u + 4grp + i for query head g*G + l16
+      if (kb + TK > kw1) {
 #pragma unroll
-      for (int o2 = 1; o2 < 64; o2 <<= 1) {
-        const int x = __shfl_up(in, o2, 64);
-        in += lane >= o2 ? x : 0;
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (kb + 16 * u + 4 * grp + i >= kw1) s[u][i] = -INFINITY;
       }
-      const uint64_t past = __builtin_amdgcn_ballot_w64(in > j);
-      if (past == 0) return;
-      const int src = __builtin_ctzll(past);
-      int k = j - __shfl(in - own, src, 64);
-      int i = 0;
-#pragma unroll
-      for (int e = 0; e < 3; ++e) {
-        const int n = __shfl(more[e], src, 64);
-        if (i == e && k >= n) {
-          k -= n;
-          ++i;
-        }
-      }
-      b = __builtin_amdgcn_readfirstlane(4 * src + i);
-      split = __builtin_amdgcn_readfirstlane(p.min_split + k);
-    }
-    pieces = pieces_of(min((clamp_len(p.lens[b]) + TK - 1) / TK, 1 << 22));
-  }
-  const int len = clamp_len(p.lens[b]);
-  if (DEAL == kDealt && p.batch * p.n_kv_heads < kFewPairs)
-    pieces = min(max(len / kPieceMinLen & ~7, p.min_split), p.n_split);  // (records merge eight at a time)
-  bf16_t *out = (bf16_t *)p.o + ((int64_t)b * p.n_heads + (int64_t)g * G) * HD;
-  const int chunk = SPLIT ? split_chunk<NW>(len, pieces) : 0;
-  const int k0 = split * chunk;
-  if (SPLIT && split > 0 && k0 >= len) return;
-  if (len == 0) {  // no key: zeros
-    for (int idx = tid; idx < G * HD; idx += 64 * NW) out[idx] = f32_to_bf16(0.f);
-    return;
-  }
-  int nw = SPLIT ? NW : WWV;  // streaming waves of this workgroup (uniform)
-  if (adapt) {
-#pragma unroll
-    for (int o2 = 32; o2 > 0; o2 >>= 1) part += __shfl_xor(part, o2, 64);
-    const int total = __builtin_amdgcn_readfirstlane(part);  // <= 512 * max_len
-    if ((int64_t)len * p.batch * 4 > (int64_t)total * 5) nw = NW;
-  }
-  // wave w < nw takes the 32-key tiles w, w + nw, w + 2*nw, ...: the waves of
-  // a workgroup stream adjacent tiles (a contiguous key range per wave, or the
-  // KV heads of one sequence placed on one XCD, measured 3-4% slower)
-  const int kw1 = SPLIT ? min(k0 + chunk, len) : len;
-  const int all_tiles = (kw1 - k0 + TK - 1) / TK;
-  const int kw0 = k0 + TK * wave;
-  const int tstride = TK * nw;  // keys between a wave's tiles
-  const int ntiles = wave < nw && all_tiles > wave ? (all_tiles - wave + nw - 1) / nw : 0;
-
-  const int64_t kv_rs = p.kv_rs;
-  const bf16_t *Kr = (const bf16_t *)p.k + b * p.kv_bs + g * p.kv_hs;
-  const bf16_t *Vr = (const bf16_t *)p.v + b * p.kv_bs + g * p.kv_hs;
-
-  dbf16x8_t qb[2];
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    if (l16 < G)
-      qb[t] = *(const dbf16x8_t *)((const bf16_t *)p.q +
-                                   ((int64_t)b * p.n_heads + g * G + l16) * HD + 8 * grp + 32 * t);
-    else
-      qb[t] = dbf16x8_t{};
-  }
-
-  // lane's 16-byte chunks of a tile: rows crow + 8i (i = 0..3), columns ccol..ccol+7
-  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-  struct RegTile {
-    u32x4 k0, k1, k2, k3, v0, v1, v2, v3;
-  };
-  const int crow = lane >> 3, ccol = (lane & 7) * 8;
-  auto gload = [&](RegTile &r, int ti) __attribute__((always_inline)) {
-    const int kb = kw0 + tstride * min(ti, ntiles - 1);  // clamped: same load count on every path
-    const int last = min(kb + TK, kw1) - 1;  // past the end: a valid row, masked to P = 0
-    const int64_t o0 = (int64_t)min(kb + crow, last) * kv_rs + ccol;
-    const int64_t o1 = (int64_t)min(kb + crow + 8, last) * kv_rs + ccol;
-    const int64_t o2 = (int64_t)min(kb + crow + 16, last) * kv_rs + ccol;
-    const int64_t o3 = (int64_t)min(kb + crow + 24, last) * kv_rs + ccol;
-    // streamed once: non-temporal loads
-    r.k0 = __builtin_nontemporal_load((const u32x4 *)(Kr + o0)); r.v0 = __builtin_nontemporal_load((const u32x4 *)(Vr + o0));
-    r.k1 = __builtin_nontemporal_load((const u32x4 *)(Kr + o1)); r.v1 = __builtin_nontemporal_load((const u32x4 *)(Vr + o1));
-    r.k2 = __builtin_nontemporal_load((const u32x4 *)(Kr + o2)); r.v2 = __builtin_nontemporal_load((const u32x4 *)(Vr + o2));
-    r.k3 = __builtin_nontemporal_load((const u32x4 *)(Kr + o3)); r.v3 = __builtin_nontemporal_load((const u32x4 *)(Vr + o3));
-  };
-  bf16_t *const kt = KT[wave], *const vt = VT[wave];
-  auto lstore = [&](const RegTile &r) __attribute__((always_inline)) {
-    *(u32x4 *)(kt + crow * WKP + ccol) = r.k0;
-    *(u32x4 *)(kt + (crow + 8) * WKP + ccol) = r.k1;
-    *(u32x4 *)(kt + (crow + 16) * WKP + ccol) = r.k2;
-    *(u32x4 *)(kt + (crow + 24) * WKP + ccol) = r.k3;
-    *(u32x4 *)(vt + crow * WKP + ccol) = r.v0;
-    *(u32x4 *)(vt + (crow + 8) * WKP + ccol) = r.v1;
-    *(u32x4 *)(vt + (crow + 16) * WKP + ccol) = r.v2;
-    *(u32x4 *)(vt + (crow + 24) * WKP + ccol) = r.v3;
-  };
-
-  float m = -INFINITY, l = 0.f;
-  df32x4_t o[4] = {df32x4_t{}, df32x4_t{}, df32x4_t{}, df32x4_t{}};
-  const float c = p.c;
-  // one 32-key tile from this wave's LDS tile; keys kb .. kb + 31
-  auto compute = [&](int kb) __attribute__((always_inline)) {
-    const bf16_t *kl = kt + 8 * grp;
-    df32x4_t s[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const bf16_t *kp = kl + (16 * u + l16) * WKP;
-      s[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const dbf16x8_t *)(kp), qb[0], df32x4_t{},
-                                                     0, 0, 0);
-      s[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const dbf16x8_t *)(kp + 32), qb[1], s[u],
-                                                     0, 0, 0);
-    }
-    // s[u][i] = score of key kb + 16u + 4grp + i for query head g*G + l16
-    if (kb + TK > kw1) {
+      float mx = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
+                       fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
+      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      const float m_new = fmaxf(m, mx);  // -inf while every key so far scores -inf
+      const float mc = (m_new == -INFINITY ? 0.f : m_new) * c;
+      const float alpha = __builtin_amdgcn_exp2f(m * c - mc);  // m = -inf -> 0
+      float rs = 0.f;
+      dbf16x8_t pb;
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (kb + 16 * u + 4 * grp + i >= kw1) s[u][i] = -INFINITY;
-    }
-    float mx = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
-                     fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float m_new = fmaxf(m, mx);  // -inf while every key so far scores -inf
-    const float mc = (m_new == -INFINITY ? 0.f : m_new) * c;
-    const float alpha = __builtin_amdgcn_exp2f(m * c - mc);  // m = -inf -> 0
-    float rs = 0.f;
-    dbf16x8_t pb;
+        for (int i = 0; i < 4; ++i) {
+          const float e = __builtin_amdgcn_exp2f(fmaf(s[u][i], c, -mc));
+          rs += e;
+          pb[4 * u + i] = (__bf16)e;  // k-slot (grp, 4u+i) = key 16u + 4grp + i
+        }
+      l = l * alpha + rs;
+      m = m_new;
+      // V^T operand: slot j of lane (grp, l16) = V[key 16(j/4) + 4grp + j%4][16dt + l16];
+      // transpose read: local lane n supplies V[key 4grp + n/4 (+16)][16dt + 4(n%4) .. +3]
+      const bf16_t *vp = vt + (4 * grp + (l16 >> 2)) * WKP + 4 * (l16 & 3);
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float e = __builtin_amdgcn_exp2f(fmaf(s[u][i], c, -mc));
-        rs += e;
-        pb[4 * u + i] = (__bf16)e;  // k-slot (grp, 4u+i) = key 16u + 4grp + i
+      for (int dt = 0; dt < 4; ++dt) {
+        o[dt] *= alpha;
+        const dbf16x4_t lo = lds_read_tr16(vp + 16 * dt);
+        const dbf16x4_t hi = lds_read_tr16(vp + 16 * WKP + 16 * dt);
+        const dbf16x8_t a = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb, o[dt], 0, 0, 0);
       }
-    l = l * alpha + rs;
-    m = m_new;
-    // V^T operand: slot j of lane (grp, l16) = V[key 16(j/4) + 4grp + j%4][16dt + l16];
-    // transpose read: local lane n supplies V[key 4grp + n/4 (+16)][16dt + 4(n%4) .. +3]
-    const bf16_t *vp = vt + (4 * grp + (l16 >> 2)) * WKP + 4 * (l16 & 3);
+    };
+
+    // The wave's tile ti goes through one register tile (loaded one tile ahead)
+    // and the wave's LDS tile.  LDS instructions of one wave execute in order,
+    // so a tile's writes follow the previous tile's reads (already consumed) and
+    // precede its own reads with no barrier; wave_barrier keeps the compiler
+    // from moving LDS accesses across.  One tile in flight per wave (4 KB of K
+    // and of V; 32 KB per CU at 4 waves) streams best: two tiles ahead measured
+    // 8% slower on config 3, more waves per workgroup slower still.
+    if (ntiles > 0) {  // wave-uniform
+      RegTile ta;
+      gload(ta, 0);
+      lstore(ta);
+      gload(ta, 1);
+      __builtin_amdgcn_wave_barrier();
+      for (int ti = 0; ti < ntiles; ++ti) {
+        compute(kw0 + tstride * ti);
+        if (ti + 1 < ntiles) {
+          __builtin_amdgcn_wave_barrier();
+          lstore(ta);
+          gload(ta, ti + 2);
+          __builtin_amdgcn_wave_barrier();
+        }
+      }
+    }
+
+    // merge the waves: o[dt][i] = O^T[d = 16dt + 4grp + i][head g*G + l16]
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (l16 < G) {
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-      o[dt] *= alpha;
-      const dbf16x4_t lo = lds_read_tr16(vp + 16 * dt);
-      const dbf16x4_t hi = lds_read_tr16(vp + 16 * WKP + 16 * dt);
-      const dbf16x8_t a = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb, o[dt], 0, 0, 0);
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) red_o[wave][l16][16 * dt + 4 * grp + i] = o[dt][i];
+      if (grp == 0) {
+        red_m[wave][l16] = m * c;  // -inf for a wave without keys
+        red_l[wave][l16] = l;
+      }
+    }
+    __syncthreads();
+    const int nvalid = pieces();
+    __builtin_assume(nvalid >= 1);
+    // query head h's record of piece n: of a dealt cache in its workgroup's second
+    // place for the cache's first piece (the workgroup's last), else in its first
+    auto rec_of = [&](int h, int n) __attribute__((always_inline)) {
+      if (DEAL == kDealt) return p.ws + ((int64_t)((2 * (bin0 + n) + (n == 0)) * p.n_kv_heads + g) * G + h) * kDecRec;
+      return p.ws + (((int64_t)b * p.n_heads + (int64_t)g * G + h) * p.n_split + n) * kDecRec;
+    };
+    for (int idx = tid; idx < G * HD; idx += 64 * NW) {
+      const int h = idx / HD, d = idx - h * HD;
+      float M = red_m[0][h];
+#pragma unroll
+      for (int w = 1; w < NW; ++w) M = fmaxf(M, red_m[w][h]);
+      const float Mu = M == -INFINITY ? 0.f : M;  // no key above -inf: every weight 0
+      float L = 0.f, A = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const float wt = __builtin_amdgcn_exp2f(red_m[w][h] - Mu);
+        L += red_l[w][h] * wt;
+        A += red_o[w][h][d] * wt;
+      }
+      if (!SPLIT || nvalid == 1) {
+        out[idx] = f32_to_bf16(L == 0.f ? 0.f : A / L);
+      } else {
+        float *rec = rec_of(h, q);
+        auto wr = [](float *q, float v) { __hip_atomic_store(q, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); };
+        wr(rec + 2 + d, A);
+        if (d == 0) {
+          wr(rec, M);
+          wr(rec + 1, L);
+        }
+      }
+    }
+    if constexpr (SPLIT) {
+      if (nvalid == 1) return;
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the record's stores have reached memory
+      __syncthreads();
+      if (tid == 0) {
+        unsigned long long *word = p.arrive_end - 2 * ((int64_t)b * p.n_kv_heads + g + 1);
+        unsigned long long old = __hip_atomic_fetch_add(word, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        bool last = old - kArrive == (unsigned long long)(nvalid - 1);
+        if (old - kArrive >= (unsigned long long)nvalid) {
+          // one split puts the tag there, then every split adds
+          old = __hip_atomic_load(word + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          while (old >> 16 != p.tag &&
+                 !__hip_atomic_compare_exchange_strong(word + 1, &old, p.tag << 16, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                       __HIP_MEMORY_SCOPE_AGENT)) {
+          }
+          const unsigned long long next =
+              __hip_atomic_fetch_add(word + 1, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+          last = (int)(next & 0xffff) == nvalid;
+          // a replay has the same tag: nothing of this count may be left for one
+          // that finds only the first word overwritten
+          if (last) __hip_atomic_store(word + 1, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (last) __hip_atomic_store(word, kArrive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last_split = last;
+      }
+      __syncthreads();
+      if (!last_split) return;
+      for (int idx = tid; idx < G * (HD / 4); idx += 64 * NW) {
+        const int h = idx / (HD / 4), d0 = 4 * (idx % (HD / 4));
+        DecMerge mg;
+        mg.start();
+        for (int s0 = 0; s0 < nvalid; s0 += 8) {
+          if constexpr (DEAL == kDealt)
+            mg.load8_from([&](int n) { return rec_of(h, n); }, nvalid, s0, d0);
+          else
+            mg.load8<true>(rec_of(h, 0), p.n_split, s0, d0);
+          mg.merge8(s0, nvalid);
+        }
+        const float4 r = mg.result();
+        const uint32_t lo = (uint32_t)f32_to_bf16(r.x) | ((uint32_t)f32_to_bf16(r.y) << 16);
+        const uint32_t hi = (uint32_t)f32_to_bf16(r.z) | ((uint32_t)f32_to_bf16(r.w) << 16);
+        bf16_t *const od = out + h * HD + d0;
+        if (((uintptr_t)out & 7) == 0) {
+          *(uint2 *)od = make_uint2(lo, hi);
+        } else {  // (o is the caller's: any element may be its first)
+          od[0] = (bf16_t)lo; od[1] = (bf16_t)(lo >> 16);
+          od[2] = (bf16_t)hi; od[3] = (bf16_t)(hi >> 16);
+        }
+      }
     }
   };
+  auto zeros = [&](int b) {  // a sequence without keys
+    bf16_t *const out = (bf16_t *)p.o + ((int64_t)b * p.n_heads + (int64_t)g * G) * HD;
+    for (int idx = tid; idx < G * HD; idx += 64 * NW) out[idx] = f32_to_bf16(0.f);
+  };
 
-  // The wave's tile ti goes through one register tile (loaded one tile ahead)
-  // and the wave's LDS tile.  LDS instructions of one wave execute in order,
-  // so a tile's writes follow the previous tile's reads (already consumed) and
-  // precede its own reads with no barrier; wave_barrier keeps the compiler
-  // from moving LDS accesses across.  One tile in flight per wave (4 KB of K
-  // and of V; 32 KB per CU at 4 waves) streams best: two tiles ahead measured
-  // 8% slower on config 3, more waves per workgroup slower still.
-  if (ntiles > 0) {  // wave-uniform
-    RegTile ta;
-    gload(ta, 0);
-    lstore(ta);
-    gload(ta, 1);
-    __builtin_amdgcn_wave_barrier();
-    for (int ti = 0; ti < ntiles; ++ti) {
-      compute(kw0 + tstride * ti);
-      if (ti + 1 < ntiles) {
-        __builtin_amdgcn_wave_barrier();
-        lstore(ta);
-        gload(ta, ti + 2);
-        __builtin_amdgcn_wave_barrier();
-      }
-    }
-  }
-
-  // merge the waves: o[dt][i] = O^T[d = 16dt + 4grp + i][head g*G + l16]
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
-  if (l16 < G) {
+  if constexpr (DEAL == kWhole) {
+    // the batch's total length (batches up to kMeanBatchMax sequences), summed
+    // by every wave itself (no barrier), read with this sequence's length
+    const bool adapt = NW > WWV && p.batch <= kMeanBatchMax;
+    int part = 0;
+    if (adapt)
+      for (int i = lane; i < p.batch; i += 64) part += clamp_len(p.lens[i]);
+    const int len = clamp_len(p.lens[bs]);
+    if (len == 0) return zeros(bs);
+    int nw = WWV;  // streaming waves of this workgroup (uniform)
+    if (adapt) {
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) red_o[wave][l16][16 * dt + 4 * grp + i] = o[dt][i];
-    if (grp == 0) {
-      red_m[wave][l16] = m * c;  // -inf for a wave without keys
-      red_l[wave][l16] = l;
+      for (int o2 = 32; o2 > 0; o2 >>= 1) part += __shfl_xor(part, o2, 64);
+      const int total = __builtin_amdgcn_readfirstlane(part);  // <= 512 * max_len
+      if ((int64_t)len * p.batch * 4 > (int64_t)total * 5) nw = NW;
     }
-  }
-  __syncthreads();
-  const int nvalid = SPLIT ? (len + chunk - 1) / chunk : 1;  // splits that hold keys
-  for (int idx = tid; idx < G * HD; idx += 64 * NW) {
-    const int h = idx / HD, d = idx - h * HD;
-    float M = red_m[0][h];
+    run(bs, 0, len, nw, [] { return 1; }, 0, 0);
+  } else if constexpr (DEAL == kSplit || DEAL == kByLength) {
+    const int b = bs / p.n_split, q = bs - b * p.n_split;
+    const int len = clamp_len(p.lens[b]);
+    // (in eights past min_split: records merge eight at a time)
+    const int pieces =
+        DEAL == kSplit ? p.n_split : min(max(len / kPieceMinLen & ~7, p.min_split), p.n_split);
+    const int chunk = split_chunk<NW>(len, pieces), k0 = q * chunk;
+    if (q > 0 && k0 >= len) return;
+    if (len == 0) return zeros(b);
+    run(b, k0, min(k0 + chunk, len), NW, [&] { return (int)((uint32_t)(len + chunk - 1) / (uint32_t)chunk); }, q, 0);
+  } else {
+    // every wave scans the batch's tiles for itself (lane: 4 sequences)
+    int t[4], own = 0, most = 0;
 #pragma unroll
-    for (int w = 1; w < NW; ++w) M = fmaxf(M, red_m[w][h]);
-    const float Mu = M == -INFINITY ? 0.f : M;  // no key above -inf: every weight 0
-    float L = 0.f, A = 0.f;
+    for (int i = 0; i < 4; ++i) {
+      const int n = 4 * lane + i < p.batch ? clamp_len(p.lens[4 * lane + i]) : 0;
+      t[i] = (n >> 5) + ((n & 31) != 0);
+      own += t[i];
+      most = max(most, t[i]);
+    }
+    static_assert(TK == 32, "tiles of 32 keys");
+    int upto = own;  // tiles of the sequences up to and with this lane's
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const float wt = __builtin_amdgcn_exp2f(red_m[w][h] - Mu);
-      L += red_l[w][h] * wt;
-      A += red_o[w][h][d] * wt;
+    for (int o2 = 1; o2 < 64; o2 <<= 1) {
+      const int x = __shfl_up(upto, o2, 64);
+      upto += lane >= o2 ? x : 0;
     }
-    if (!SPLIT || nvalid == 1) {
-      out[idx] = f32_to_bf16(L == 0.f ? 0.f : A / L);
-    } else {
-      float *rec = p.ws + (((int64_t)b * p.n_heads + (int64_t)g * G + h) * p.n_split + split) * kDecRec;
-      auto wr = [](float *q, float v) { __hip_atomic_store(q, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); };
-      wr(rec + 2 + d, A);
-      if (d == 0) {
-        wr(rec, M);
-        wr(rec + 1, L);
-      }
+    const int total = __builtin_amdgcn_readlane(upto, 63);
+    most = wave_max_i32(most);
+    for (int b = bs; b < p.batch; b += p.groups)
+      if (clamp_len(p.lens[b]) == 0) zeros(b);
+    const int share = max((int)((uint32_t)total / (uint32_t)p.groups) + 1, kShareMin);
+    // Equal pieces (min_split a cache) end with the longest cache's.  Where that
+    // isn't far past a share, they take less time than shares over the ends of
+    // caches and the merges that those need: with 0 / 32 / 48 / 80 in kUneven's
+    // place, 86 batches of 65..128 pairs and 6000..9000 rows took 0.83 / 0.77 /
+    // 0.78 / 0.85 of the former chunk kernel's time, 22 short caches (13..829 keys,
+    // 8 KV heads) 14.8 / 9.5 / 9.5 / 9.5 us.
+    if (most <= (share + max(share / 4, kUneven)) * (int64_t)p.min_split) {
+      const int b = bs / p.min_split, q = bs - b * p.min_split;
+      const int len = b < p.batch ? clamp_len(p.lens[b]) : 0;
+      const int chunk = split_chunk<NW>(len, p.min_split), k0 = q * chunk;
+      auto n = [&] { return (int)((uint32_t)(len + chunk - 1) / (uint32_t)chunk); };
+      if (k0 < len) run(b, k0, min(k0 + chunk, len), NW, n, q, b * p.min_split);
+      return;
     }
-  }
-  if constexpr (SPLIT) {
-    if (nvalid == 1) return;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the record's stores have reached memory
-    __syncthreads();
-    if (tid == 0) {
-      unsigned long long *word = p.arrive_end - 2 * ((int64_t)b * p.n_kv_heads + g + 1);
-      unsigned long long old = __hip_atomic_fetch_add(word, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      bool last = old - kArrive == (unsigned long long)(nvalid - 1);
-      if (old - kArrive >= (unsigned long long)nvalid) {
-        // one split puts the tag there, then every split adds
-        old = __hip_atomic_load(word + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        while (old >> 16 != p.tag &&
-               !__hip_atomic_compare_exchange_strong(word + 1, &old, p.tag << 16, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                     __HIP_MEMORY_SCOPE_AGENT)) {
+    const int end = min((bs + 1) * share, total);
+    for (int pos = bs * share; pos < end;) {
+      const int src = __builtin_ctzll(__builtin_amdgcn_ballot_w64(upto > pos));
+      int b = 4 * src, first = __builtin_amdgcn_readlane(upto - own, src);  // b's first tile
+      int tb = __builtin_amdgcn_readlane(t[0], src);
+#pragma unroll
+      for (int i = 1; i < 4; ++i) {
+        const int ti = __builtin_amdgcn_readlane(t[i], src);
+        if (pos >= first + tb) {
+          first += tb;
+          tb = ti;
+          ++b;
         }
-        const unsigned long long next =
-            __hip_atomic_fetch_add(word + 1, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
-        last = (int)(next & 0xffff) == nvalid;
-        // a replay has the same tag: nothing of this count may be left for one
-        // that finds only the first word overwritten
-        if (last) __hip_atomic_store(word + 1, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
-      if (last) __hip_atomic_store(word, kArrive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      last_split = last;
-    }
-    __syncthreads();
-    if (!last_split) return;
-    for (int idx = tid; idx < G * (HD / 4); idx += 64 * NW) {
-      const int h = idx / (HD / 4), d0 = 4 * (idx % (HD / 4));
-      const float *rec = p.ws + ((int64_t)b * p.n_heads + (int64_t)g * G + h) * p.n_split * kDecRec;
-      DecMerge mg;
-      mg.start();
-      for (int s0 = 0; s0 < nvalid; s0 += 8) {
-        mg.load8<true>(rec, p.n_split, s0, d0);
-        mg.merge8(s0, nvalid);
-      }
-      const float4 r = mg.result();
-      const uint32_t lo = (uint32_t)f32_to_bf16(r.x) | ((uint32_t)f32_to_bf16(r.y) << 16);
-      const uint32_t hi = (uint32_t)f32_to_bf16(r.z) | ((uint32_t)f32_to_bf16(r.w) << 16);
-      bf16_t *const od = out + h * HD + d0;
-      if (((uintptr_t)out & 7) == 0) {
-        *(uint2 *)od = make_uint2(lo, hi);
-      } else {  // (o is the caller's: any element may be its first)
-        od[0] = (bf16_t)lo; od[1] = (bf16_t)(lo >> 16);
-        od[2] = (bf16_t)hi; od[3] = (bf16_t)(hi >> 16);
-      }
+      const int stop = min(first + tb, end), len = clamp_len(p.lens[b]);
+      const int bin0 = (int)((uint32_t)first / (uint32_t)share);
+      auto n = [&] { return (int)((uint32_t)(first + tb - 1) / (uint32_t)share) - bin0 + 1; };
+      run(b, TK * (pos - first), min(TK * (stop - first), len), NW, n, bs - bin0, bin0);
+      pos = stop;
+      __syncthreads();  // the next piece's LDS writes follow this one's reads
     }
   }
 }
@@ -1401,35 +1425,35 @@ uint32_t next_plan_epoch() {
 int whole_splits(int units, int max_len) {
   return std::max(1, std::min({256 / units, 8, (max_len + 127) / 128 - 1}));
 }
-// Where caches can be longer than those lines were drawn for, their pieces
-// follow the lengths (kDealt).  Returns the most pieces of a cache, and in more
-// the workgroups per KV head for pieces past whole_splits(), in outliers whether only a
-// cache of more than four times the batch's mean length has any; 0: equal
-// pieces as above.  us, former chunk kernel / equal pieces / dealt, 4 KV heads:
-//  - below 32 pairs (a piece per 1024 keys, in eights since eight records merge
-//    at a time): one cache of 16384 keys 23.4 / 16.8 / 13.4, of 131072 86 / 94 /
-//    32, with 8 KV heads 74 / 97 / 44; of 1543 in 131072 rows 11.8 / 6.9 / 6.9
-//  - to 128 pairs, from 16384 rows: one cache of 32768 among 31 of 500 65 / 95 /
-//    21, 12 token-major caches of 913..32149 56 / 49 / 50 (every cache dealt:
-//    53); where the equal pieces leave a fifth of 256 workgroups unused every
-//    cache is dealt: 24 of 2308..30794 96 / 102 / 70 (32 of 816..30488, which
-//    leave none: 119 / 113 / 162).  32 of 562..16351 57 / 60 / 61 is left.
-//  - to 255 pairs, from 5120 rows: 33 token-major caches of 639..8162 47 / 53 /
-//    32, all of 8192 61 / 58 / 58, 40 of 888..16067 85 / 102 / 71, 56 of
-//    549..5949 39 / 43 / 42; one of 16384 among 39 of 500 42 / 94 / 15.  Eight
-//    waves hold a CU each even where they find no piece, so head-major calls
-//    have 64 workgroups for them (256 cost 63 uniform caches 2.5%): one of 16384
-//    among 39 of 500 45 / 73 / 20.
-// The scan costs 0.6 us: 8 caches of 16384 23.3 / 23.9, 63 of 1000 in 16384 rows
-// 12.6 / 14.2 (99 before).
-int dealt_splits(int batch, int n_kv_heads, int max_len, bool token_major, int *more, int *outliers) {
-  const int units = batch * n_kv_heads, by_len = max_len / kPieceMinLen;
-  *more = *outliers = 0;
-  if (batch > kDealtMax || units >= 256 || by_len < (units > 128 ? 5 : 16)) return 0;
-  if (units < kFewPairs) return std::min({256 / units, 64, by_len & ~7});
-  *more = (units > 128 && !token_major ? 64 : 256) / n_kv_heads;
-  *outliers = units <= 128 && units * whole_splits(units, max_len) > 204;
-  return *more ? std::min(by_len, units > 128 ? 32 : 64) : 0;
+// Where caches can be longer than those lines were drawn for:
+//  - below 32 pairs a cache's pieces follow its own length (the most of them
+//    returned, 0: equal pieces as above): a piece per 1024 keys.  us, former chunk
+//    kernel / equal pieces / by length, 4 KV heads: one cache of 16384 keys 23.4
+//    / 16.8 / 13.4, of 131072 86 / 94 / 32, with 8 KV heads 74 / 97 / 44; of 1543
+//    in 131072 rows 11.8 / 6.9 / 6.9
+int pieces_by_length(int units, int max_len) {
+  return units < 32 && max_len >= 16384 ? std::min({256 / units, 64, max_len / kPieceMinLen & ~7}) : 0;
+}
+//  - from there the batch's tiles are dealt in equal shares (kDealt) to the
+//    workgroups per KV head returned (0: as above), one per compute unit.  1500
+//    drawn batches in both layouts (equal, ragged and mixed lengths, one long
+//    cache, all short), equal pieces / dealt as ratios to the former chunk kernel,
+//    mean and worst: 65..255 pairs from 8192 rows 1.08 and 4.4 / 0.72 and 1.04, of
+//    4096..8191 0.85 and 2.6 / 0.77 and 1.18, of 2500..4095 0.74 and 1.65 / 0.77
+//    and 1.31; 32..64 pairs from 20000 rows 0.80 and 1.78 / 0.74 and 1.03, of
+//    10240..19999 0.70 and 1.28 / 0.70 and 1.01, of 4000..6999 0.63 and 0.91 /
+//    0.69 and 0.98.  us, chunk kernel / equal pieces / dealt, 4 KV heads: 33
+//    token-major caches of 707..8103 keys 48 / 51 / 32, all of 8192 61 / 58 / 49, 40
+//    of 1269..16128 91 / 104 / 66, 32 of 618..15604 58 / 58 / 46, 24 of 4079..30201
+//    102 / 103 / 75, one of 16384 among 39 of 500 53 / 92 / 19.  The scan over the
+//    lengths costs 0.6 us: 8 of 16384 34.7 / 23.9 / 24.5.
+int dealt_groups(int batch, int n_kv_heads, int max_len) {
+  const int64_t units = (int64_t)batch * n_kv_heads;
+  // a lane scans four sequences (units < 256), and tiles are counted in 31 bits
+  if (units < 32 || units >= 256 || (int64_t)batch * max_len > ((int64_t)1 << 34)) return 0;
+  // Two records a workgroup, at most 512 / n_kv_heads of a head, and the arrival
+  // words fit the 128-key chunks' workspace: over 2000 / n_kv_heads records.
+  return max_len >= (units > 64 ? 4096 : 10240) ? 256 / n_kv_heads : 0;
 }
 // a launch's 48-bit tag: a mixed counter (SplitMix64's finaliser), so that
 // no plausible memory contents look like this launch's arrivals
@@ -1575,15 +1599,14 @@ int gqa_decode_impl(int dtype, const void *q, const void *k_cache, const void *v
                                         std::to_string((size_t)BN_GQA_DECODE_SCRATCH_BYTES) +
                                         "-byte scratch");
   size_t words = 0;
-  bool dealt = false;
   if (bsplit) {  // (the no-allocation limit above stays that of the chunks' partials)
-    p.min_split = p.n_split = whole_splits(batch * n_kv_heads, max_len);
-    const int most =
-        dealt_splits(batch, n_kv_heads, max_len, p.kv_rs != HD, &p.more, &p.outliers);
-    dealt = most > p.n_split;
-    if (dealt) p.n_split = most;
-    words = p.n_split > 1 ? (size_t)batch * n_kv_heads * 16 + 8 : 0;
-    need = p.n_split > 1 ? (size_t)batch * n_heads * p.n_split * kDecRec * sizeof(float) + words : 0;
+    const int units = batch * n_kv_heads;
+    p.min_split = whole_splits(units, max_len);
+    p.n_split = std::max(p.min_split, pieces_by_length(units, max_len));
+    p.groups = dealt_groups(batch, n_kv_heads, max_len);
+    const size_t records = p.groups ? 2 * p.groups * (size_t)n_heads : (size_t)batch * n_heads * p.n_split;
+    words = p.groups || p.n_split > 1 ? (size_t)units * 16 + 8 : 0;
+    need = words ? records * kDecRec * sizeof(float) + words : 0;
   }
   int st = ensure_device();
   if (st) return st;
@@ -1607,15 +1630,14 @@ int gqa_decode_impl(int dtype, const void *q, const void *k_cache, const void *v
       p.arrive_end = (unsigned long long *)(((uintptr_t)ws + bytes) & ~(uintptr_t)7);
       p.tag = next_split_tag();
     }
-    const int units = batch * n_kv_heads;
-    const dim3 grid((unsigned)(dealt && p.more ? units * p.min_split + n_kv_heads * p.more : units * p.n_split));
-    const bool eight = dealt ? units > 128 && p.kv_rs == HD : p.n_split == 1;  // waves
+    const dim3 grid((unsigned)(p.groups ? p.groups * n_kv_heads : batch * n_kv_heads * p.n_split));
+    const bool by_length = p.n_split > p.min_split, eight = !p.groups && p.n_split == 1;  // (waves)
 #define BN_SPLIT(GG)                                                                                        \
   do {                                                                                                      \
-    if (dealt && eight)                                                                                     \
-      hipLaunchKernelGGL((decode_bf16_whole_kernel<GG, WW1, kDealt>), grid, dim3(64 * WW1), 0, s, p);       \
-    else if (dealt)                                                                                         \
+    if (p.groups)                                                                                           \
       hipLaunchKernelGGL((decode_bf16_whole_kernel<GG, WWV, kDealt>), grid, dim3(64 * WWV), 0, s, p);       \
+    else if (by_length)                                                                                     \
+      hipLaunchKernelGGL((decode_bf16_whole_kernel<GG, WWV, kByLength>), grid, dim3(64 * WWV), 0, s, p);    \
     else if (eight)                                                                                         \
       hipLaunchKernelGGL((decode_bf16_whole_kernel<GG, WW1, kSplit>), grid, dim3(64 * WW1), 0, s, p);       \
     else                                                                                                    \

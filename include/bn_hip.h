@@ -338,7 +338,7 @@ int bn_llama_decode(const bn_llama_config *config, const float *embed,
  * bn_gqa_decode_workspace_size() bytes (NULL: taken from the pool when the
  * call needs it); single-pass calls use none: bf16 caches of at most 256 keys
  * or with batch*n_kv_heads at least the device's compute units, or above half
- * of them with max_len below 5120.  Other bf16 calls keep split records there and, at its end, arrival
+ * of them with max_len below 4096.  Other bf16 calls keep split records there and, at its end, arrival
  * words that the splits count in on, two per (sequence, KV head).  A pair
  * finds its words ready if an earlier call with this workspace (same address
  * and size) split that pair and nothing has written over them since; on any

@@ -836,16 +836,23 @@ def test_decode_bf16_keys_of_minus_infinity(case, mask):
 
 
 # bf16 caches whose pieces follow the lengths: a few pairs (pieces by a cache's own length, past one group of
-# eight records), up to 128 pairs (outliers alone, or every cache where workgroups are left) and up to 255 (whole
-# caches, the longer ones in pieces), in both layouts, with empty and one-key caches
+# eight records), and batches of 32 to 255 pairs dealt in equal shares (a workgroup's share within one cache, over
+# the ends of several, past the batch's end; even batches in equal pieces), in both layouts, with empty and
+# one-key caches
 DEALT_DECODE_CASES = [
     # lengths, max_len, H, Hkv, head-major
     ([16384], 16384, 8, 1, False),
     ([20000, 0, 9000], 20480, 16, 4, True),                          # 12 pairs
     ([16000] * 5, 16400, 8, 4, False),                               # 20 pairs: twelve pieces at most
-    ([500] * 5 + [16384] + [1, 0] + [700] * 4, 16384, 32, 4, True),  # 48 pairs, an outlier
+    ([16385] * 8, 16400, 32, 4, False),                              # 32 pairs of one length
+    ([500] * 5 + [16384] + [1, 0] + [700] * 4, 16384, 32, 4, True),  # 48 pairs, one long cache
     ([9000 + 600 * i for i in range(12)], 16384, 32, 4, False),      # the same, none
-    ([3, 0, 16384, 2000] * 6, 16384, 8, 4, False),                   # 96 pairs: every cache
+    ([3, 0, 16384, 2000] * 6, 16384, 8, 4, False),                   # 96 pairs
+    ([4609, 0] + [1] * 15, 4700, 16, 4, True),                       # 68 pairs: three pieces a cache, just too uneven
+    ([4608, 0] + [1] * 15, 4700, 16, 4, True),                       # and just even enough
+    ([1537, 0] + [1] * 32, 4096, 16, 4, False),                      # 136 pairs, whole: the same
+    ([1536, 0] + [1] * 32, 4096, 16, 4, False),
+    ([0] * 17, 4096, 8, 4, False),                                   # no keys at all
     ([0] * 10 + [6000] + [400] * 22, 6000, 32, 4, False),            # 132 pairs
     (list(range(100, 6100, 150)), 6100, 16, 4, False),               # 160 pairs
     ([0] * 62 + [9000], 9000, 8, 4, True),                           # 252 pairs, one cache with keys
@@ -879,7 +886,8 @@ def test_decode_bf16_pieces_by_length(case):
                 rows = slice(h * G, (h + 1) * G)
                 s = q[b, rows].double() @ k[b, :lens[b], h].double().T * 0.125
                 ref[b, rows] = torch.softmax(s, 1) @ v[b, :lens[b], h].double()
-        assert_close(host(o[ld > 0]), ref[ld > 0].cpu().numpy(), BF16_TOL, f"{what} {case}")
+        if any(lens):
+            assert_close(host(o[ld > 0]), ref[ld > 0].cpu().numpy(), BF16_TOL, f"{what} {case}")
         assert not o[ld == 0].any()
 
     def run():
